@@ -17,6 +17,7 @@
 #include "kgh_kernels.h"
 
 #include <climits>
+#include <cstdint>
 
 namespace {
 
@@ -500,8 +501,200 @@ __global__ __launch_bounds__(FA_THREADS, 1) void flashAttentionKernel(const half
   }
 }
 
-// Attention without matrix cores, for fp32 contexts and head shapes the
-// kernel above does not take: one thread per (board, head, query), two
+// ---------------------------------------------------------------------------
+// fp32 attention on the matrix cores (v_mfma_f32_32x32x2f32), for the head
+// shapes of the fp16 kernel and any number of keys. A workgroup of four
+// wave64s takes 128 queries of one (board, query head); K and V of its kv
+// head stream through LDS in chunks of 64 keys, two buffers, the next
+// chunk's rows loading into registers during the current one's work. Wave w
+// owns queries 32w.. and computes S^T = K Q^T (lane = query) for the chunk's
+// two 32-key tiles, an online softmax per lane, and O^T += V^T P^T, with P
+// taken straight from the accumulator registers: register r of the two lane
+// halves holds keys k(r) and k(r) + 4, which is one K = 2 step of the second
+// product when V is read at those two keys.
+// Bound: the matrix cores (64 cycles per 32x32x2 step; 4096 cycles per 32x32
+// tile of scores at dims 64/64). Eight boards of 19x19, six heads of 64: 42 us
+// per launch against 7.70 ms on one thread per query (whose 128 output
+// accumulators live in scratch memory).
+constexpr int AF_THREADS = 256;
+constexpr int AF_QUERIES = 128;
+constexpr int AF_KEYS = 64;
+
+template<int DQ, int DV>
+__global__ __launch_bounds__(AF_THREADS) void attentionF32Kernel(const float* __restrict__ qkv, int ld, int kOff, int vOff, int H, int KV,
+                                                                const float* __restrict__ mask, int HW, float* __restrict__ out,
+                                                                int ldOut, float scale, int queryBlocks) {
+  static_assert(DQ % 8 == 0 && DV % 4 == 0 && DQ <= 64 && DV <= 64, "head dims");
+  constexpr int DVP = (DV + 31) / 32 * 32;
+  constexpr int KLD = DQ + 4;  // floats per K row (16-byte pad: the 16 rows of a ds_read_b128 phase in distinct banks)
+  __shared__ __attribute__((aligned(16))) float Ks[2][AF_KEYS * KLD];
+  __shared__ __attribute__((aligned(16))) float Vs[2][AF_KEYS * DVP];
+  __shared__ float keyBias[2][AF_KEYS];  // 0 for a valid key, -inf for a masked one or one past HW
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int laneRow = lane & 31;
+  const int half = lane >> 5;
+  const int item = blockIdx.x / queryBlocks;
+  const int n = item / H;
+  const int h = item - n * H;
+  const int kvh = h / (H / KV);
+  const size_t rowBase = (size_t)n * HW;
+  const int qi = (blockIdx.x - item * queryBlocks) * AF_QUERIES + (tid >> 6) * 32 + laneRow;
+  const int qRow = qi < HW ? qi : HW - 1;
+
+  // Thread tid moves K 16-byte groups and V 16-byte groups tid + it *
+  // AF_THREADS of a chunk; rows of masked keys, keys past HW and dims past DV
+  // are zero.
+  constexpr int K_VECS = AF_KEYS * (DQ / 4), V_VECS = AF_KEYS * (DVP / 4);
+  constexpr int K_ITERS = K_VECS / AF_THREADS, V_ITERS = V_VECS / AF_THREADS;
+  static_assert(K_ITERS * AF_THREADS == K_VECS && V_ITERS * AF_THREADS == V_VECS, "staging loops without a remainder");
+  floatx4 kRows[K_ITERS], vRows[V_ITERS];
+  float kOn[K_ITERS], vOn[V_ITERS], keyOn = 0.0f;
+  auto fetch = [&](int key0) {
+#pragma unroll
+    for(int it = 0; it < K_ITERS; it++) {
+      const int i = tid + it * AF_THREADS;
+      const int key = key0 + i / (DQ / 4);
+      const size_t row = rowBase + min(key, HW - 1);
+      kRows[it] = *(const floatx4*)(qkv + row * ld + kOff + kvh * DQ + (i % (DQ / 4)) * 4);
+      kOn[it] = key < HW ? mask[row] : 0.0f;
+    }
+#pragma unroll
+    for(int it = 0; it < V_ITERS; it++) {
+      const int i = tid + it * AF_THREADS;
+      const int key = key0 + i / (DVP / 4);
+      const int d = (i % (DVP / 4)) * 4;
+      const size_t row = rowBase + min(key, HW - 1);
+      vRows[it] = *(const floatx4*)(qkv + row * ld + vOff + kvh * DV + (d < DV ? d : 0));
+      vOn[it] = key < HW && d < DV ? mask[row] : 0.0f;
+    }
+    if(tid < AF_KEYS) keyOn = key0 + tid < HW ? mask[rowBase + key0 + tid] : 0.0f;
+  };
+  const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto stage = [&](int buf) {
+#pragma unroll
+    for(int it = 0; it < K_ITERS; it++) {
+      const int i = tid + it * AF_THREADS;
+      *(floatx4*)&Ks[buf][i / (DQ / 4) * KLD + (i % (DQ / 4)) * 4] = kOn[it] != 0.0f ? kRows[it] : +zero;
+    }
+#pragma unroll
+    for(int it = 0; it < V_ITERS; it++) {
+      const int i = tid + it * AF_THREADS;
+      *(floatx4*)&Vs[buf][i * 4] = vOn[it] != 0.0f ? vRows[it] : +zero;
+    }
+    if(tid < AF_KEYS) keyBias[buf][tid] = keyOn != 0.0f ? 0.0f : -INFINITY;
+  };
+
+  // Query fragments: dims 8g + 4 half + 0..3 of this lane's query, the
+  // order in which K is read.
+  floatx4 qf[DQ / 8];
+#pragma unroll
+  for(int g = 0; g < DQ / 8; g++) qf[g] = *(const floatx4*)(qkv + (rowBase + qRow) * ld + h * DQ + g * 8 + half * 4);
+  const float on = mask[rowBase + qRow];
+  fetch(0);
+
+  floatx16 o[DVP / 32];
+#pragma unroll
+  for(int db = 0; db < DVP / 32; db++)
+#pragma unroll
+    for(int r = 0; r < 16; r++) o[db][r] = 0.0f;
+  // Scores stay unscaled (scale > 0 keeps their order): p = 2^((s - mRun) c).
+  const float c = scale * 1.44269504088896341f;
+  float mRun = -INFINITY, lRun = 0.0f;
+  stage(0);
+  __syncthreads();
+  const int chunks = (HW + AF_KEYS - 1) / AF_KEYS;
+  for(int ch = 0; ch < chunks; ch++) {
+    const int buf = ch & 1;
+    if(ch + 1 < chunks) fetch((ch + 1) * AF_KEYS);
+    floatx16 s[2];
+#pragma unroll
+    for(int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for(int r = 0; r < 16; r++) s[kt][r] = 0.0f;
+    // The two tiles' chains interleave.
+#pragma unroll
+    for(int g = 0; g < DQ / 8; g++) {
+      floatx4 a[2];
+#pragma unroll
+      for(int kt = 0; kt < 2; kt++) a[kt] = *(const floatx4*)&Ks[buf][(kt * 32 + laneRow) * KLD + g * 8 + half * 4];
+#pragma unroll
+      for(int j = 0; j < 4; j++)
+#pragma unroll
+        for(int kt = 0; kt < 2; kt++) s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[kt][j], qf[g][j], s[kt], 0, 0, 0);
+    }
+    float m = -INFINITY;
+#pragma unroll
+    for(int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for(int r = 0; r < 16; r++) {
+        s[kt][r] += keyBias[buf][kt * 32 + (r >> 2) * 8 + half * 4 + (r & 3)];
+        m = fmaxf(m, s[kt][r]);
+      }
+    m = fmaxf(m, __shfl_xor(m, 32));
+    // While a query has seen no valid key, mRun stays -inf and every p is 0
+    // (masked scores are -inf); the factor of the first valid chunk is 0 on
+    // accumulators that are still 0.
+    const float mNew = fmaxf(mRun, m);
+    const float ref = mNew == -INFINITY ? 0.0f : mNew;
+    const float corr = __builtin_amdgcn_exp2f((mRun - ref) * c);
+    mRun = mNew;
+    float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for(int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for(int r = 0; r < 16; r++) {
+        const float p = __builtin_amdgcn_exp2f((s[kt][r] - ref) * c);
+        s[kt][r] = p;
+        part[r & 3] += p;
+      }
+    float psum = (part[0] + part[1]) + (part[2] + part[3]);
+    psum += __shfl_xor(psum, 32);
+    lRun = lRun * corr + psum;
+#pragma unroll
+    for(int db = 0; db < DVP / 32; db++)
+#pragma unroll
+      for(int r = 0; r < 16; r++) o[db][r] *= corr;
+#pragma unroll
+    for(int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for(int r = 0; r < 16; r++) {
+        const int key = kt * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
+#pragma unroll
+        for(int db = 0; db < DVP / 32; db++)
+          o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(Vs[buf][key * DVP + db * 32 + laneRow], s[kt][r], o[db], 0, 0, 0);
+      }
+    // The other buffer was last read before the previous barrier.
+    if(ch + 1 < chunks) stage(buf ^ 1);
+    __syncthreads();
+  }
+
+  if(qi < HW) {
+    const float invL = on != 0.0f && lRun > 0.0f ? 1.0f / lRun : 0.0f;
+    float* dst = out + (rowBase + qi) * ldOut + h * DV;
+#pragma unroll
+    for(int db = 0; db < DVP / 32; db++)
+#pragma unroll
+      for(int g = 0; g < 4; g++) {
+        const int d = db * 32 + g * 8 + half * 4;
+        if(d < DV)
+          *(float4*)(dst + d) = make_float4(o[db][4 * g] * invL, o[db][4 * g + 1] * invL, o[db][4 * g + 2] * invL, o[db][4 * g + 3] * invL);
+      }
+  }
+}
+
+template<int DQ, int DV>
+void launchAttentionF32(const float* qkv, int ld, int kOff, int vOff, int H, int KV, const float* mask, int HW, int batch, float* out,
+                        int ldOut, float scale, hipStream_t stream) {
+  const int queryBlocks = (HW + AF_QUERIES - 1) / AF_QUERIES;
+  hipLaunchKernelGGL((attentionF32Kernel<DQ, DV>), dim3((unsigned)batch * H * queryBlocks), dim3(AF_THREADS), 0, stream, qkv, ld, kOff, vOff,
+                     H, KV, mask, HW, out, ldOut, scale, queryBlocks);
+  KGH_CHECK_LAUNCH();
+}
+
+// Attention without matrix cores, for head shapes the kernels above do not
+// take: one thread per (board, head, query), two
 // passes over the keys as in the reference.
 template<typename T>
 __global__ void attentionSimpleKernel(const T* __restrict__ qkv, int ld, int kOff, int vOff, int H, int KV, int dq, int dv,
@@ -664,6 +857,18 @@ void launchAttention(T* qkv, int ld, int kOff, int vOff, int H, int KV, int dq, 
   if(done) return;
   // Plain path: rotate Q and K in place, then attend.
   if(cosT != nullptr) launchRope<T>(qkv, ld, H, KV, dq, cosT, sinT, learnable, HW, batch * HW, stream);
+  if constexpr(sizeof(T) == 4) {
+    // 16-byte rows; every batch size takes the same kernel, so a board's
+    // outputs do not depend on its batch.
+    const bool aligned = ld % 4 == 0 && kOff % 4 == 0 && vOff % 4 == 0 && ldOut % 4 == 0 && (((uintptr_t)qkv | (uintptr_t)out) & 15) == 0 &&
+                         (long)batch * H * ((HW + AF_QUERIES - 1) / AF_QUERIES) < INT_MAX;
+    if(aligned && ((dq == 64 && dv == 64) || (dq == 32 && (dv == 32 || dv == 16)))) {
+      if(dq == 64) launchAttentionF32<64, 64>(qkv, ld, kOff, vOff, H, KV, mask, HW, batch, out, ldOut, scale, stream);
+      else if(dv == 32) launchAttentionF32<32, 32>(qkv, ld, kOff, vOff, H, KV, mask, HW, batch, out, ldOut, scale, stream);
+      else launchAttentionF32<32, 16>(qkv, ld, kOff, vOff, H, KV, mask, HW, batch, out, ldOut, scale, stream);
+      return;
+    }
+  }
   const long total = (long)batch * H * HW;
   hipLaunchKernelGGL(attentionSimpleKernel<T>, dim3((unsigned)((total + 127) / 128)), dim3(128), 0, stream, qkv, ld, kOff, vOff, H, KV,
                      dq, dv, mask, HW, batch, out, ldOut, scale);
