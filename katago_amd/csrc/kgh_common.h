@@ -288,7 +288,9 @@ struct BoardGeom {
 
 // Kernel choices for one conv launch: the autotuner's search space. All of
 // them sum the K dimension in the same order, so they give bitwise the same
-// results. CONV_AUTO is the built-in heuristic.
+// results. CONV_AUTO is the built-in heuristic. Saved tuning tables hold these
+// numbers: new kernels are appended, and one that is gone (CONV_RETIRED_*)
+// applies to no shape, so a table that names it runs the built-in choice.
 enum ConvVariant {
   CONV_AUTO = 0,
   CONV_TW_192,    // 3x3 fp16 tap-window DMA kernel, 12 waves, 192 output channels per tile
@@ -309,12 +311,18 @@ enum ConvVariant {
   CONV_DMA1H_192,  // 1x1 fp16 DMA kernel with 192-row tiles, two workgroups per CU
   CONV_DMA1H_128,
   CONV_DMA1H_64,
-  CONV_BOARD_HALF_64,  // the one-board kernel on half a board per workgroup (two per CU), 64 output channels per tile
-  CONV_ALLK1_64,  // 1x1 fp16 kernel for small row counts: 64-row tiles, every input channel in LDS at once
-  CONV_ALLK1_32,
+  CONV_RETIRED_19,
+  CONV_RETIRED_20,
+  CONV_ALLK1_32,  // 1x1 fp16 kernel for small row counts: 64-row tiles, every input channel in LDS at once
   CONV_DMA1_256_GLU,  // 1x1 fp16 DMA kernel, 384 x 256 tiles, gated (SwiGLU) epilogue only
-  CONV_BOARD_HALF_64_T32,  // the half-board kernel with 32-row wave tiles (12 waves per workgroup)
-  CONV_BOARD_HALF_192,  // the half-board kernel with 192 output channels per tile (one workgroup per CU)
+  CONV_RETIRED_23,
+  CONV_RETIRED_24,
+  CONV_STREAM3_32,  // 3x3 fp16 streamed-weight kernel (any board size), 32 rows x 64 output channels per tile
+  CONV_STREAM3_64,
+  CONV_STREAM3_128,
+  CONV_STREAM3_192,
+  CONV_STREAM1_32,  // the same for 1x1
+  CONV_STREAM1_64,
   CONV_VARIANT_COUNT
 };
 

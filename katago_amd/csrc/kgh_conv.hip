@@ -15,6 +15,7 @@
 // double-buffered, with the next step's global loads issued before the
 // current step's matrix-core work.
 #include "kgh_conv_device.h"
+#include "kgh_conv_stream.h"
 
 #include <climits>
 #include <cstdio>
@@ -1690,15 +1691,15 @@ void launchTapWindow(const half_t* x, int cinStride, int cinPad, int cout, const
   KGH_CHECK_LAUNCH();
 }
 
-template<int BN, int RW = BW_ROW_WAVES, int WT = BW_WTM>
+template<int BN>
 void launchBoardWindow(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
                        const ConvEpilogue<half_t>& epi, hipStream_t stream) {
-  static const std::string name = kernelLabel("convBoardWindowKernel<3x3 fp16, BN=%d, %s, %d-row wave tiles>", BN,
-                                              RW == BW_ROW_WAVES ? "one board per workgroup" : "half a board per workgroup", WT);
+  static const std::string name = kernelLabel("convBoardWindowKernel<3x3 fp16, BN=%d, one board per workgroup, %d-row wave tiles>",
+                                              BN, BW_WTM);
   kgh::g_lastConvKernel = name.c_str();
-  dim3 grid(g.batch * (RW == BW_ROW_WAVES ? 1 : 2) * (cout / BN));
-  hipLaunchKernelGGL((convBoardWindowKernel<BN, BN == 64 ? 9 : 6, false, RW, WT>), grid, dim3(128 * RW * BW_WTM / WT), 0, stream, x,
-                     cinStride, cinPad, cout, w, g.batch, epi);
+  dim3 grid(g.batch * (cout / BN));
+  hipLaunchKernelGGL((convBoardWindowKernel<BN, BN == 64 ? 9 : 6>), grid, dim3(128 * BW_ROW_WAVES), 0, stream, x, cinStride, cinPad,
+                     cout, w, g.batch, epi);
   KGH_CHECK_LAUNCH();
 }
 
@@ -1738,42 +1739,53 @@ template<>
 bool dispatchTapWindow<half_t>(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
                                const ConvEpilogue<half_t>& epi, hipStream_t stream) {
   const long M = (long)g.batch * g.H * g.W;
-  // One board per workgroup. The widest column tile while it gives at least
-  // 160 workgroups; below that, 64-column tiles (the most workgroups), but
-  // not for the stem (one 32-channel chunk), which the tuner keeps on the
-  // tile kernel. Tuner measurements: at 128 boards the 64-column tiles take
-  // b10c128's convs in 23-26 us vs 29-33 us, b18c384nbt's in 50-55 us vs
-  // 52-57 us; at 192 boards the wide tiles win; at 1 to 96 boards the
-  // 64-column tiles beat the 128-row tile kernel by 1.5-2x.
-  if(boardWindowFits(cinStride, cinPad, cout, 64, g, epi)) {
-    const int wide = cout % 192 == 0 ? 192 : cout % 128 == 0 ? 128 : 64;
-    if((long)g.batch * (cout / wide) >= 160) {
-      if(wide == 192) launchBoardWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream);
-      else if(wide == 128) launchBoardWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
-      else launchBoardWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
+  // 19x19 boards, one per workgroup with 192- or 128-column tiles, where those
+  // fill at least three quarters of their rounds of the 256 CUs: b18c384nbt's
+  // 192 -> 192 convs 58.8 us at 200 boards and 67 us at 256, against 57.9 and
+  // 74 us on the streamed kernel; 54.4 against 49.5 us at 160 boards, where
+  // 96 CUs idle. With 64-column tiles (320 -> 320 channels, 160 boards) one
+  // takes 143 us, the streamed kernel 119.
+  const bool board = boardWindowFits(cinStride, cinPad, cout, 64, g, epi);
+  const int wide = cout % 192 == 0 ? 192 : cout % 128 == 0 ? 128 : 64;
+  const long boards = (long)g.batch * (cout / wide);
+  if(board && wide > 64 && boards >= 192 * ((boards + 255) / 256)) {
+    if(wide == 192) launchBoardWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else launchBoardWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    return true;
+  }
+  const int tile = kgh::streamTile3x3(cinStride, cinPad, cout, g, epi);
+  if(tile != CONV_AUTO) {
+    kgh::launchStream(tile, x, cinStride, cinPad, cout, w, g, epi, stream);
+    return true;
+  }
+  // Too many input channels for two streamed 128-row windows per CU or one of
+  // 192 rows (above about 320), and more than one round of smaller tiles. At
+  // 19x19, one board per workgroup from 128 of its 64-column tiles (384 -> 384
+  // at 40 boards: forwards of six blocks 636 us, 689 on streamed 128-row tiles;
+  // 512 -> 512 at 24: 706, 824 on half boards, 921 on streamed 64-row tiles).
+  // Else the largest streamed tile that fits, and the tap-window kernel where
+  // that is 64 rows and there are 128 of its row tiles (512 channels, 300
+  // boards 13x13: 301 us; at 100 boards 64 streamed rows take 115 us, the
+  // 128-row tile kernel 201).
+  if(board && (long)g.batch * (cout / 64) >= 128) {
+    if(boards >= 160 && wide == 192) launchBoardWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else if(boards >= 160 && wide == 128) launchBoardWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else launchBoardWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    return true;
+  }
+  for(int v : {CONV_STREAM3_128, CONV_STREAM3_64, CONV_STREAM3_32}) {
+    if(v != CONV_STREAM3_128 && M >= 128L * TW_BM && tapWindowFits(cinStride, cinPad, cout, 64, g, epi)) {
+      if(wide == 192) launchTapWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream);
+      else if(wide == 128) launchTapWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
+      else launchTapWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
       return true;
     }
-    if(cinPad >= 64) {
-      // Half boards with 32-row wave tiles (12 waves, one workgroup per CU)
-      // while the half boards fit the CUs one to a CU; half boards with
-      // 96-row tiles (two workgroups per CU) up to one and a half rounds of
-      // the CUs' 512 slots (the tuner's pick over whole boards for C2's net
-      // at 96 and 128 boards: 40 vs 45 us per conv).
-      const long halves = (long)g.batch * 2 * (cout / 64);
-      if(halves <= 256) launchBoardWindow<64, 2, 32>(x, cinStride, cinPad, cout, w, g, epi, stream);
-      else if(halves <= 768) launchBoardWindow<64, 2>(x, cinStride, cinPad, cout, w, g, epi, stream);
-      else launchBoardWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    if(kgh::streamFits(v, cinStride, cinPad, cout, g, epi)) {
+      kgh::launchStream(v, x, cinStride, cinPad, cout, w, g, epi, stream);
       return true;
     }
   }
-  if(g.W + 1 > TW_PAD_MAX || cinPad % 32 != 0 || cinStride % 8 != 0 || epi.maskResidualAdd) return false;
-  if(M < 128L * TW_BM) return false;
-  if(M * cinStride >= (1L << 31) || 9L * cout * cinPad >= (1L << 31)) return false;
-  if(cout % 192 == 0) launchTapWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream);
-  else if(cout % 128 == 0) launchTapWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
-  else if(cout % 64 == 0) launchTapWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
-  else return false;
-  return true;
+  return false;
 }
 
 // 384 x 256 tiles for gated (SwiGLU) convs only: at 256 columns the
@@ -1814,15 +1826,13 @@ bool allK1x1Fits(int cinStride, int cinPad, int cout, int bn, BoardGeom g) {
   return dma1x1Fits(cinStride, cinPad, cout, bn, g) && cinPad <= 32 * SMALL1_MAX_STEPS;
 }
 
-template<int BN>
-void launch1x1AllK(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
-                   const ConvEpilogue<half_t>& epi, hipStream_t stream) {
-  static const std::string name = kernelLabel("conv1x1AllKKernel<1x1 fp16, BN=%d>", BN);
-  kgh::g_lastConvKernel = name.c_str();
+void launch1x1AllK(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g, const ConvEpilogue<half_t>& epi,
+                   hipStream_t stream) {
+  kgh::g_lastConvKernel = "conv1x1AllKKernel<1x1 fp16, BN=32>";
   const int M = g.batch * g.H * g.W;
-  dim3 grid((M + SMALL1_BM - 1) / SMALL1_BM * (cout / BN)), block(BN / 32 * 128);
-  if(epi.glu) hipLaunchKernelGGL((conv1x1AllKKernel<BN, true>), grid, block, 0, stream, x, cinStride, cinPad, cout, w, g, epi);
-  else hipLaunchKernelGGL((conv1x1AllKKernel<BN, false>), grid, block, 0, stream, x, cinStride, cinPad, cout, w, g, epi);
+  dim3 grid((M + SMALL1_BM - 1) / SMALL1_BM * (cout / 32)), block(128);
+  if(epi.glu) hipLaunchKernelGGL((conv1x1AllKKernel<32, true>), grid, block, 0, stream, x, cinStride, cinPad, cout, w, g, epi);
+  else hipLaunchKernelGGL((conv1x1AllKKernel<32, false>), grid, block, 0, stream, x, cinStride, cinPad, cout, w, g, epi);
   KGH_CHECK_LAUNCH();
 }
 
@@ -1838,21 +1848,22 @@ bool dispatch1x1Dma<half_t>(const half_t* x, int cinStride, int cinPad, int cout
   const long M = (long)g.batch * g.H * g.W;
   if(cinPad % 32 != 0 || cinStride % 8 != 0) return false;
   if(M * cinStride >= (1L << 31) || (long)cout * cinPad >= (1L << 31)) return false;
+  const int tile = kgh::streamTile1x1(cinStride, cinPad, cout, g, epi);
+  if(tile != CONV_AUTO) {
+    kgh::launchStream(tile, x, cinStride, cinPad, cout, w, g, epi, stream);
+    return true;
+  }
   // Too few 384-row tiles to fill most CUs: from 24 tiles of 192 rows, the
-  // 192-row kernel with 64-column tiles (two workgroups per CU; the tuner
-  // picks it for b18c384nbt's 1x1 convs at 16 to 64 boards, 12-20 us vs
-  // 18-24 us on the 128-row tile kernel). Below that, the whole-K kernel
-  // (one memory round trip per tile; C2's net at 1-8 boards: forwards
-  // 0.09-0.12 ms shorter than on the 128-row tile kernel), with 32-column
-  // tiles while 64-column ones would give fewer than 64 workgroups; else
-  // the tile kernel.
+  // 192-row kernel with 64-column tiles (two workgroups per CU; b18c384nbt's
+  // 1x1 convs at 16 to 64 boards 12-20 us vs 18-24 us on the 128-row tile
+  // kernel). Below that, where the streamed kernel does not apply, the whole-K
+  // kernel (one memory round trip per tile; b18c384nbt at 1-8 boards: forwards
+  // 0.09-0.12 ms shorter than on the 128-row tile kernel); else the tile
+  // kernel.
   if((M + TW_BM - 1) / TW_BM * (cout / 64) < 3 * 128) {
     if(M < 24L * 192) {
       if(!allK1x1Fits(cinStride, cinPad, cout, 32, g)) return false;
-      if(cout % 64 == 0 && (M + SMALL1_BM - 1) / SMALL1_BM * (cout / 64) >= 64)
-        launch1x1AllK<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
-      else
-        launch1x1AllK<32>(x, cinStride, cinPad, cout, w, g, epi, stream);
+      launch1x1AllK(x, cinStride, cinPad, cout, w, g, epi, stream);
       return true;
     }
     if(cout % 64 != 0) return false;
@@ -1881,9 +1892,8 @@ bool variantFits(int v, int ky, int cinStride, int cinPad, int cout, BoardGeom g
       if(v == CONV_TW_64) return tapWindowFits(cinStride, cinPad, cout, 64, g, epi);
       if(v == CONV_BOARD_192) return boardWindowFits(cinStride, cinPad, cout, 192, g, epi);
       if(v == CONV_BOARD_128) return boardWindowFits(cinStride, cinPad, cout, 128, g, epi);
-      if(v == CONV_BOARD_64 || v == CONV_BOARD_HALF_64 || v == CONV_BOARD_HALF_64_T32)
-        return boardWindowFits(cinStride, cinPad, cout, 64, g, epi);
-      if(v == CONV_BOARD_HALF_192) return boardWindowFits(cinStride, cinPad, cout, 192, g, epi);
+      if(v == CONV_BOARD_64) return boardWindowFits(cinStride, cinPad, cout, 64, g, epi);
+      if(v >= CONV_STREAM3_32 && v <= CONV_STREAM3_192) return kgh::streamFits(v, cinStride, cinPad, cout, g, epi);
     }
     else {
       if(v == CONV_DMA1_192) return dma1x1Fits(cinStride, cinPad, cout, 192, g);
@@ -1892,9 +1902,9 @@ bool variantFits(int v, int ky, int cinStride, int cinPad, int cout, BoardGeom g
       if(v == CONV_DMA1H_192) return dma1x1Fits(cinStride, cinPad, cout, 192, g);
       if(v == CONV_DMA1H_128) return dma1x1Fits(cinStride, cinPad, cout, 128, g);
       if(v == CONV_DMA1H_64) return dma1x1Fits(cinStride, cinPad, cout, 64, g);
-      if(v == CONV_ALLK1_64) return allK1x1Fits(cinStride, cinPad, cout, 64, g);
       if(v == CONV_ALLK1_32) return allK1x1Fits(cinStride, cinPad, cout, 32, g);
       if(v == CONV_DMA1_256_GLU) return epi.glu && dma1x1Fits(cinStride, cinPad, cout, 256, g);
+      if(v == CONV_STREAM1_32 || v == CONV_STREAM1_64) return kgh::streamFits(v, cinStride, cinPad, cout, g, epi);
     }
   }
   else {
@@ -1932,11 +1942,7 @@ void launchVariant(int v, int ky, const T* x, int cinStride, int cinPad, int cou
       case CONV_BOARD_192: launchBoardWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
       case CONV_BOARD_128: launchBoardWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
       case CONV_BOARD_64: launchBoardWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
-      case CONV_BOARD_HALF_64: launchBoardWindow<64, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
-      case CONV_BOARD_HALF_64_T32: launchBoardWindow<64, 2, 32>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
-      case CONV_BOARD_HALF_192: launchBoardWindow<192, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
-      case CONV_ALLK1_64: launch1x1AllK<64>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
-      case CONV_ALLK1_32: launch1x1AllK<32>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
+      case CONV_ALLK1_32: launch1x1AllK(x, cinStride, cinPad, cout, w, g, epi, stream); return;
       case CONV_DMA1_192: launch1x1Dma<192>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
       case CONV_DMA1_128: launch1x1Dma<128>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
       case CONV_DMA1_64: launch1x1Dma<64>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
@@ -1945,6 +1951,10 @@ void launchVariant(int v, int ky, const T* x, int cinStride, int cinPad, int cou
       case CONV_DMA1H_64: launch1x1Dma<64, 192>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
       case CONV_DMA1_256_GLU: launch1x1DmaGlu256(x, cinStride, cinPad, cout, w, g, epi, stream); return;
       default: break;
+    }
+    if(v >= CONV_STREAM3_32 && v <= CONV_STREAM1_64) {
+      kgh::launchStream(v, x, cinStride, cinPad, cout, w, g, epi, stream);
+      return;
     }
   }
   throw KghError(5, "conv: variant does not apply");
@@ -1988,7 +1998,8 @@ const char* convVariantName(int variant) {
   static const char* names[] = {"auto", "tw192", "tw128", "tw64", "tw8w192", "dma1x1_192", "dma1x1_128", "dma1x1_64",
                                 "tile192", "tile128", "tile96", "tile64", "tile32", "board192", "board128", "board64",
                                 "dma1x1h_192", "dma1x1h_128", "dma1x1h_64", "boardhalf64", "allk1x1_64", "allk1x1_32",
-                                "dma1x1_256glu", "boardhalf64t32", "boardhalf192"};
+                                "dma1x1_256glu", "boardhalf64t32", "boardhalf192",
+                                "stream3_32", "stream3_64", "stream3_128", "stream3_192", "stream1_32", "stream1_64"};
   static_assert(sizeof(names) / sizeof(names[0]) == CONV_VARIANT_COUNT, "a name per variant");
   return variant >= 0 && variant < CONV_VARIANT_COUNT ? names[variant] : "?";
 }
@@ -2117,11 +2128,14 @@ void launchConvSplitK(const half_t* x, int cinStride, int cinPad, int cout, cons
   KGH_CHECK_LAUNCH();
 }
 
+bool fragWeights(int ky, int kx, int cinPad, int cout) {
+  return ky == kx && (ky == 1 || ky == 3) && cinPad % 32 == 0 && cout % 32 == 0;
+}
 bool f32SplitWeights(int ky, int kx, int cinPad, int cout) { return ky == 3 && kx == 3 && cinPad % 16 == 0 && cout % 32 == 0; }
 
 size_t preparedConvWeightElems(bool fp16, int ky, int kx, int cout, int cinPad) {
   const size_t n = (size_t)ky * kx * cout * cinPad;
-  return !fp16 && f32SplitWeights(ky, kx, cinPad, cout) ? 2 * n : n;
+  return (fp16 ? fragWeights(ky, kx, cinPad, cout) : f32SplitWeights(ky, kx, cinPad, cout)) ? 2 * n : n;
 }
 
 template<typename T>
@@ -2130,6 +2144,11 @@ void prepareConvWeights(const float* dW, T* dOut, int cout, int cin, int cinPad,
   hipLaunchKernelGGL(prepareConvWeightsKernel<T>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, dW, dOut, cout,
                      cin, cinPad, ky, kx);
   KGH_CHECK_LAUNCH();
+  if constexpr(std::is_same<T, half_t>::value) {
+    if(fragWeights(ky, kx, cinPad, cout)) {
+      prepareFragWeights(dW, dOut + total, cout, cin, cinPad, ky, stream);
+    }
+  }
   if constexpr(std::is_same<T, float>::value) {
     if(f32SplitWeights(ky, kx, cinPad, cout)) {
       hipLaunchKernelGGL(prepareF32SplitWeightsKernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, dW,
