@@ -323,6 +323,11 @@ enum ConvVariant {
   CONV_STREAM3_192,
   CONV_STREAM1_32,  // the same for 1x1
   CONV_STREAM1_64,
+  CONV_SPLIT3_32,  // 3x3 fp32 on bf16 matrix cores, 32-row tiles
+  CONV_SPLIT3_64,
+  CONV_SPLIT3_96,
+  CONV_SPLIT1_K,     // the same for 1x1, K over the waves
+  CONV_SPLIT1_WIDE,  // columns over the waves
   CONV_VARIANT_COUNT
 };
 

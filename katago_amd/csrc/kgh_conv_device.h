@@ -38,16 +38,6 @@ template<> struct MfmaCfg<half_t> {
   }
 };
 
-template<> struct MfmaCfg<float> {
-  static constexpr int BK = 16;
-  static constexpr int KSUB = 2;
-  static constexpr int LANE_K = 1;
-  typedef float Frag;
-  __device__ static floatx16 mma(Frag a, Frag b, floatx16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-  }
-};
-
 constexpr int CONV_BM = 128;
 constexpr int CONV_THREADS = 256;
 constexpr int CONV_STAGE_LD = 36;  // fp32 row stride of the epilogue's accumulator stage
