@@ -287,6 +287,18 @@ __device__ void poolBoardVec(const T* __restrict__ g, int ld, int C, const float
   }
 }
 
+// Reads one float of every 128-byte line of p[0 .. n) into registers, so that
+// weights used later in the kernel are on their way to this XCD's L2 (a
+// forward of b18c384nbt reads more weights than the L2s hold, so they come
+// from memory each time). The sum keeps the loads alive; the caller passes it
+// to touchDone once there is nothing else to wait for.
+__device__ __forceinline__ float touchLines(const float* __restrict__ p, int n) {
+  float t = 0.0f;
+  for(int i = threadIdx.x * 32; i < n; i += blockDim.x * 32) t += p[i];
+  return t;
+}
+__device__ __forceinline__ void touchDone(float t) { asm volatile("" ::"v"(t)); }
+
 // out[co] = sum_i pooled[i] * W[i][co] over cin inputs, as four consecutive
 // segments of the inputs (one thread each, all their weight loads in
 // flight) added in order: the same order at any block size, so the fused
@@ -349,7 +361,15 @@ __global__ __launch_bounds__(POOL_THREADS) void poolVecKernel(const T* __restric
 // BN + activation of the board's regular channels with the bias from LDS:
 // bitwise the outputs of those two launches, without the bias round trip
 // through global memory and the second launch.
+//
+// gridDim.y workgroups share a board: each pools it and forms the bias (one
+// memory round trip and a short matvec), then activates its share of the
+// rows, which is what one workgroup spends half its time on (a board of 361 x
+// 128 mish is 46 thousand activations on one CU). As many as fit the 256 CUs
+// one to a CU, at most eight: b18c384nbt at one board 17.9 -> 13.1 us per
+// launch, 16 boards 18.7 -> 13.2, b10c128 at 64 boards 17.5 -> 12.7.
 constexpr int GPOOL_ACT_THREADS = 512;
+constexpr int GPOOL_MAX_PARTS = 8;
 template<typename T, int ACT>
 __global__ __launch_bounds__(GPOOL_ACT_THREADS) void gpoolBiasActKernel(GpoolBiasActArgs<T> a) {
   constexpr int VEC = 16 / (int)sizeof(T);
@@ -361,9 +381,11 @@ __global__ __launch_bounds__(GPOOL_ACT_THREADS) void gpoolBiasActKernel(GpoolBia
   float* pooled = maxs + C;           // [3C]
   float* nb = pooled + 3 * C;         // [cout]
   float* red = nb + a.cout;           // [2 * blockDim.x * VEC], then [2 * blockDim.x]
+  const float touched = touchLines(a.Wt, 3 * C * a.cout);
   // Eight positions in flight: at 512 threads twelve would not fit the
   // 256 registers per lane.
   poolBoardVec<T, 8>(a.g, a.ldG, C, a.mask, n, a.HW, sums, maxs, red, red + 2 * GPOOL_ACT_THREADS * VEC);
+  touchDone(touched);
   const float div = a.maskSum[n];
   const float sq = sqrtf(div) - 14.0f;
   for(int c = threadIdx.x; c < C; c += blockDim.x) {
@@ -377,9 +399,10 @@ __global__ __launch_bounds__(GPOOL_ACT_THREADS) void gpoolBiasActKernel(GpoolBia
   __syncthreads();
   // Twelve 16-byte rows in flight per thread (one round at C2's 361 x 128).
   const int CG = a.cout / VEC;
-  const int items = a.HW * CG;
+  const int share = (a.HW * CG + gridDim.y - 1) / gridDim.y;
+  const int items = min(a.HW * CG, (int)(blockIdx.y + 1) * share);
   constexpr int U = 12;
-  for(int it0 = threadIdx.x; it0 < items; it0 += U * blockDim.x) {
+  for(int it0 = blockIdx.y * share + threadIdx.x; it0 < items; it0 += U * blockDim.x) {
     T in[U][VEC];
 #pragma unroll
     for(int u = 0; u < U; u++) {
@@ -469,9 +492,14 @@ __global__ __launch_bounds__(HEADVEC_THREADS) void headVectorKernel(HeadVectorAr
   int maxCout = max(max(a.p1C, a.passC), max(a.policyC, a.v2C));
   maxCout = max(maxCout, max(3, a.scoreC));
   float* red = part + max(HEADVEC_THREADS, maxCout);
+  float touched = touchLines(a.g1W, 3 * a.g1C * a.p1C) + touchLines(a.v2W, 3 * a.v1C * a.v2C) +
+                  touchLines(a.v3W, a.v2C * 3) + touchLines(a.sv3W, a.v2C * a.scoreC);
+  if(a.pass2W != nullptr) touched += touchLines(a.passW, 3 * a.g1C * a.passC) + touchLines(a.pass2W, a.passC * a.policyC);
+  else touched += touchLines(a.passW, 3 * a.g1C * a.policyC);
   // Eight positions in flight: at 512 threads twelve would not fit the
   // 256 registers per lane.
   poolBoardVec<T, 8>(a.gv, a.ldGv, C, a.mask, n, a.HW, sums, maxs, red, red + 2 * HEADVEC_THREADS * VEC);
+  touchDone(touched);
   // poolRowsGPool (eigenbackend.cpp:152-177) for g1, poolRowsValueHead
   // (eigenbackend.cpp:179-197) for v1.
   const float div = a.maskSum[n];
@@ -896,7 +924,7 @@ void launchGpoolBiasAct(const GpoolBiasActArgs<T>& a, hipStream_t stream) {
   if(!gpoolBiasActApplies(a)) throw KghError(5, "gpool bias/activation kernel: shapes not supported");
   constexpr int VEC = 16 / (int)sizeof(T);
   const size_t smem = (size_t)(5 * a.C + a.cout + 2 * GPOOL_ACT_THREADS * VEC + 2 * GPOOL_ACT_THREADS) * sizeof(float);
-  const dim3 grid(a.batch), block(GPOOL_ACT_THREADS);
+  const dim3 grid(a.batch, std::min(std::max(256 / a.batch, 1), GPOOL_MAX_PARTS)), block(GPOOL_ACT_THREADS);
   switch(a.act) {
     case KGH_ACT_IDENTITY: hipLaunchKernelGGL((gpoolBiasActKernel<T, KGH_ACT_IDENTITY>), grid, block, smem, stream, a); break;
     case KGH_ACT_RELU: hipLaunchKernelGGL((gpoolBiasActKernel<T, KGH_ACT_RELU>), grid, block, smem, stream, a); break;
