@@ -194,7 +194,7 @@ def latency(h, call, lm, cfg, batch=1, steps=200):
     out = {"hbm_resident_ms": {"p50": q(lat, 50), "p90": q(lat, 90), "min": q(lat, 0)},
            "pcie_inclusive_ms": host_path(False)}
     if cfg.fp16 and batch <= 16:
-        # The same with hipLowLatency (split-K 3x3 convs): device-resident
+        # The same with hipLowLatency: device-resident
         # inputs on a one-row device handle, and the host-memory path.
         h.set_low_latency(True)
         for _ in range(5):
@@ -209,8 +209,7 @@ def latency(h, call, lm, cfg, batch=1, steps=200):
         h.set_low_latency(False)
         out["low_latency"] = {"hbm_resident_ms": {"p50": q(fast, 50), "p90": q(fast, 90), "min": q(fast, 0)},
                               "pcie_inclusive_ms": host_path(True),
-                              "what": "hipLowLatency: split-K 3x3 convolutions (up to 8 workgroups per board and 64 "
-                                      "output channels, fp32 partial sums added in a fixed order)"}
+                              "what": "hipLowLatency (the default kernels)"}
     out.update({"forwards": steps, "what": "one board per forward, host wall clock from launch to synchronize"})
     return out
 
@@ -339,7 +338,7 @@ def main():
     ap.add_argument("--latency", action="store_true", help="also time single forwards (always on at --batch 1)")
     ap.add_argument("--no-latency", action="store_true", help="skip the single-forward timing even at --batch 1")
     ap.add_argument("--low-latency", action="store_true",
-                    help="run the timed forwards in the handle's low-latency mode (split-K 3x3 convs; batch <= 16)")
+                    help="run the timed forwards in the handle's low-latency mode (batch <= 16)")
     ap.add_argument("--no-serve", action="store_true",
                     help="skip the PCIe-inclusive measurement through the batching evaluator")
     ap.add_argument("--copy-calibration", type=int, default=0, metavar="MIB",
