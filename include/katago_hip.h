@@ -254,11 +254,17 @@ int kgh_handle_set_tuning(kgh_handle* handle, const char* table);
 int kgh_handle_get_tuning(kgh_handle* handle, char* buf, int32_t buflen);
 
 /* Low-latency mode for small batches (config key hipLowLatency of the
- * NeuralNet backend; no counterpart in nninterface.h). It once ran 3x3 convs
- * split-K over several workgroups; the default kernels are now faster at every
- * batch it takes (b18c384nbt, one board: 0.86 ms by default, 1.10 ms split-K),
- * so the mode is accepted as before, for handles of max_batch <=
- * KGH_LOW_LATENCY_MAX_BATCH, and runs them. */
+ * NeuralNet backend; no counterpart in nninterface.h): every fp16 3x3 conv of
+ * more than 384 input channels on 19x19 boards that the one-board kernel takes
+ * runs split-K (below that the default kernels are faster), its 32-channel
+ * chunks spread over up to eight workgroups per (board, 64 output channels)
+ * whose fp32 partial sums a second kernel adds in a fixed order before the
+ * epilogue.
+ * Results are deterministic and independent of the batch size within the
+ * mode, but not bitwise equal to the default kernels (other summation order;
+ * both stay within the fp16 tolerances of the oracle). Only for handles of
+ * max_batch <= KGH_LOW_LATENCY_MAX_BATCH; enabling allocates the partial-sum
+ * buffer (8 * max_batch * nn_x * nn_y * widest channel count floats). */
 #define KGH_LOW_LATENCY_MAX_BATCH 16
 int kgh_handle_set_low_latency(kgh_handle* handle, int32_t enabled);
 

@@ -51,8 +51,8 @@ void* kgn_create_context_ex(void* loaded_model, int32_t nn_x, int32_t nn_y, int3
 
 /* createComputeContext with a ConfigParser holding the given "key = value"
  * lines ('#' starts a comment), as they would appear in a KataGo config file:
- * hipAutoTune, hipTunerFile, hipLowLatency (handles of nnMaxBatchSize
- * <= 16, see kgh_handle_set_low_latency). */
+ * hipAutoTune, hipTunerFile, hipLowLatency (split-K 3x3 convolutions for
+ * handles of nnMaxBatchSize <= 16, see kgh_handle_set_low_latency). */
 void* kgn_create_context_cfg(void* loaded_model, int32_t nn_x, int32_t nn_y, int32_t use_fp16, const char* home_data_dir,
                              const char* config, char* err, int32_t errlen);
 

@@ -588,6 +588,11 @@ struct kgh_handle {
   bool graphsEnabled = true;
   std::vector<GraphEntry> graphs;
 
+  // Low-latency mode (kgh_handle_set_low_latency): the 3x3 convs the split-K
+  // path takes run with their fp32 partial sums in splitWork.
+  bool lowLatency = false;
+  float* splitWork = nullptr;
+
   // Autotuned kernel variant per conv shape, keyed by (ky, kx, cinPad, cout,
   // M, gated epilogue, residual, masked residual); every conv launch of a
   // forward looks its shape up here (kgh_handle_autotune, kgh_handle_set_tuning).
@@ -710,6 +715,14 @@ struct Runner {
   }
 
   void conv(const ConvW& c, const T* x, int ldx, const ConvEpilogue<T>& e) {
+    if constexpr(std::is_same<T, half_t>::value) {
+      if(h != nullptr && h->lowLatency && kgh::convSplitKApplies(ldx, c.cinPad, c.cout, c.ky, c.kx, c.wPrep, g, e)) {
+        ProfRec* rec = profStart(c);
+        kgh::launchConvSplitK((const half_t*)x, ldx, c.cinPad, c.cout, (const half_t*)c.wPrep, g, e, h->splitWork, s);
+        profStop(rec);
+        return;
+      }
+    }
     int variant = CONV_AUTO;
     if(h != nullptr) {
       const kgh_handle::TuneKey key = {c.ky, c.kx, c.cinPad, c.cout, M, e.glu, e.residual != nullptr ? 1 : 0, e.maskResidualAdd};
@@ -2137,6 +2150,16 @@ int kgh_handle_set_low_latency(kgh_handle* handle, int32_t enabled) {
     requireHandle(handle);
     if(enabled && handle->maxBatch > KGH_LOW_LATENCY_MAX_BATCH)
       invalid("low-latency mode takes handles of max_batch <= " + std::to_string(KGH_LOW_LATENCY_MAX_BATCH));
+    if(enabled && handle->splitWork == nullptr) {
+      // Up to eight splits of the widest activation of the net.
+      const Net& net = handle->model->net;
+      int maxC = std::max(net.tmpC, 1);
+      for(int c : net.depthC) maxC = std::max(maxC, c);
+      KGH_HIP_CHECK(hipSetDevice(handle->model->device));
+      handle->splitWork = handle->arena.allocN<float>((size_t)8 * handle->maxBatch * handle->H * handle->W * maxC);
+    }
+    handle->lowLatency = enabled != 0;
+    dropGraphs(handle);
   });
 }
 

@@ -363,6 +363,18 @@ bool convRopeOk(int cinStride, int cinPad, int cout, int ky, int kx, const void*
 template<typename T>
 bool convNormFoldOk(int cinStride, int cinPad, int cout, int ky, int kx, const void* wPrepared, const ConvEpilogue<T>& epi);
 
+// Split-K form of the one-board 3x3 kernel for small batches (the handle's
+// low-latency mode): the conv's 32-channel chunks are spread over up to eight
+// workgroups per (board, 64-column tile), whose fp32 partial sums
+// (convSplitKWorkFloats floats of work) a second kernel adds in a fixed order
+// before applying the epilogue. Deterministic, but not bitwise equal to the
+// other kernels (different summation order).
+bool convSplitKApplies(int cinStride, int cinPad, int cout, int ky, int kx, const void* wPrepared, BoardGeom g,
+                       const ConvEpilogue<half_t>& epi);
+size_t convSplitKWorkFloats(int cinPad, int cout, BoardGeom g);
+void launchConvSplitK(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
+                      const ConvEpilogue<half_t>& epi, float* work, hipStream_t stream);
+
 // Converts fp32 weights (oc, ic, y, x) to the kernel layout [tap][oc][cinPad]
 // of type T on device (zero-padded channels).
 template<typename T>

@@ -679,16 +679,107 @@ constexpr int BW_BM = 384;
 constexpr int BW_WTM = BW_BM / BW_ROW_WAVES;           // 96 rows per wave
 constexpr int BW_MAX_CIN = 1024;
 
+constexpr int SPLITK_BN = 64;
+constexpr int SPLITK_MAX_SPLITS = 8;
+
 // Zero source of the window's border and gap slots (zero-initialised at load;
 // never written). Long enough for every chunk offset up to BW_MAX_CIN.
 __device__ __attribute__((aligned(256))) half_t kZeroChannels[BW_MAX_CIN + 64];
 
-template<int BN, int NB>
-__global__ __launch_bounds__(128 * BW_ROW_WAVES, 1) void convBoardWindowKernel(const half_t* __restrict__ x, int cinStride, int cinPad,
-                                                                              int cout, const half_t* __restrict__ w,
-                                                                              ConvEpilogue<half_t> epi) {
-  constexpr int RW = BW_ROW_WAVES;
-  constexpr int WT = BW_WTM;
+
+// Sums split-K partials work[s][m][c0..c0+7] over s = 0, 1, ... in order
+// (all loads issued first), then applies the epilogue contract to the sums.
+template<int ACT>
+__device__ __forceinline__ void splitKEpilogue8(const float* __restrict__ work, int splits, int M, int HW, int cout,
+                                                const ConvEpilogue<half_t>& epi, int m, int c0) {
+  // Every load first (partials, residual, mask, per-channel parameters): one
+  // memory round trip per thread.
+  const bool hasRes = epi.residual != nullptr;
+  const bool hasAct = epi.outAct != nullptr && c0 >= epi.actBegin;
+  const int ca = hasAct ? c0 - epi.actBegin : 0;
+  const uint4 raw = hasRes ? *(const uint4*)(epi.residual + (size_t)m * epi.ldRes + c0) : make_uint4(0, 0, 0, 0);
+  const float msk = epi.mask[m];
+  // (The parameter arrays are only 4-byte aligned: scalar loads.)
+  float s8[8], b8[8];
+  if(hasAct) {
+#pragma unroll
+    for(int k = 0; k < 8; k++) {
+      s8[k] = epi.actScale[ca + k];
+      b8[k] = epi.actBias[ca + k];
+    }
+  }
+  float4 part[2 * SPLITK_MAX_SPLITS];
+#pragma unroll
+  for(int s = 0; s < SPLITK_MAX_SPLITS; s++)
+    if(s < splits) {
+      const float4* p = (const float4*)(work + ((size_t)s * M + m) * cout + c0);
+      part[2 * s] = p[0];
+      part[2 * s + 1] = p[1];
+    }
+  float v[8];
+#pragma unroll
+  for(int k = 0; k < 8; k++) v[k] = 0.0f;
+#pragma unroll
+  for(int s = 0; s < SPLITK_MAX_SPLITS; s++)
+    if(s < splits) {
+      const float4 a = part[2 * s], b = part[2 * s + 1];
+      v[0] += a.x;
+      v[1] += a.y;
+      v[2] += a.z;
+      v[3] += a.w;
+      v[4] += b.x;
+      v[5] += b.y;
+      v[6] += b.z;
+      v[7] += b.w;
+    }
+  if(epi.ncBias != nullptr) {
+    const float* nb = epi.ncBias + (size_t)(m / HW) * epi.ldNC + c0;
+#pragma unroll
+    for(int k = 0; k < 8; k++) v[k] += nb[k];
+  }
+  if(hasRes) {
+    const half_t* rv = (const half_t*)&raw;
+#pragma unroll
+    for(int k = 0; k < 8; k++) v[k] = epi.maskResidualAdd ? (float)rv[k] + v[k] * msk : (float)rv[k] + v[k];
+  }
+  if(c0 < epi.rawEnd) {
+    half_t o[8];
+#pragma unroll
+    for(int k = 0; k < 8; k++) o[k] = (half_t)v[k];
+    *(uint4*)(epi.outRaw + (size_t)m * epi.ldRaw + c0) = *(const uint4*)o;
+  }
+  if(hasAct) {
+    half_t o[8];
+#pragma unroll
+    for(int k = 0; k < 8; k++) o[k] = (half_t)(kgh_activate_fast(v[k] * s8[k] + b8[k], ACT) * msk);
+    *(uint4*)(epi.outAct + (size_t)m * epi.ldAct + ca) = *(const uint4*)o;
+  }
+}
+
+// SPLIT: split-K for small batches. Workgroup (board, column tile, split s)
+// runs only the 32-channel chunks of split s (gridDim.y splits) and stores
+// its fp32 accumulators to work[s][m][cout] (board rows only); the residual
+// and the epilogue are left to splitKEpilogueKernel, which sums the splits in
+// order. (Summing in the last split to finish instead, behind device-scope
+// fences, measured twice as slow: each fence writes back and invalidates the
+// XCD's whole L2.)
+//
+// RW = 2: half a board per workgroup (rows 0..191 or 192..383 of the board's
+// 384, with a window of the 13 padded rows they reach), 2 row waves and 2
+// column waves, two workgroups per CU: twice the workgroups at small and
+// middle batches. Every output sums the same products in the same order as
+// with RW = 4, so the two are bitwise equal.
+//
+// WT = 32: wave tiles of 32 rows instead of 96, three times the waves (12
+// per half board) for the same work: the RW loader waves of each kind still
+// issue every DMA, the others only compute, and each SIMD holds three waves
+// to hide the per-step latencies that bound small and middle batches (LDS
+// fragment reads per matrix instruction 2 instead of 4/3). The sums are the
+// same, in the same order: bitwise equal to WT = 96.
+template<int BN, int NB, bool SPLIT = false, int RW = BW_ROW_WAVES, int WT = BW_WTM>
+__global__ __launch_bounds__(128 * RW * BW_WTM / WT, RW == BW_ROW_WAVES || WT != BW_WTM ? 1 : 2) void convBoardWindowKernel(
+    const half_t* __restrict__ x, int cinStride, int cinPad, int cout, const half_t* __restrict__ w, int batch,
+    ConvEpilogue<half_t> epi, float* __restrict__ work = nullptr) {
   // NB weight buffers, loaded LA = NB - 3 steps ahead: the DMA for step
   // s + LA goes to buffer (s - 3) mod NB, free once step s - 1's barrier is
   // passed. Nine buffers (six steps ahead) for 64-column tiles, whose small
@@ -704,14 +795,20 @@ __global__ __launch_bounds__(128 * BW_ROW_WAVES, 1) void convBoardWindowKernel(c
   // vs 68.4 us), +8% at 8-32 boards.
   constexpr int TPB = 3;
   constexpr int WTN = BN / 2;
+  static_assert(WT == BW_WTM || WT == 32, "wave tiles of 96 or 32 rows");
   constexpr int RB = WT / 32;
   constexpr int CB = WTN / 32;
-  constexpr int NW = 2 * RW;
+  constexpr int CW = RW * BW_WTM / WT;  // row waves that compute (RW of them also load)
+  constexpr int NW = 2 * CW;
   static_assert(WTN % 32 == 0, "wave tile must be a multiple of 32 columns");
+  static_assert(RW == BW_ROW_WAVES || RW == 2, "a whole board or half of one");
   constexpr int B_PER = BN / 16 / RW;
   static_assert(B_PER * 16 * RW == BN, "weights split evenly over the weight waves");
-  constexpr int WIN_PER = BW_WIN_PER;
-  constexpr int WIN_BYTES = BW_WIN_BYTES;
+  // Window: all 21 padded rows, or the 13 that half a board's taps reach.
+  constexpr int WROWS = RW == BW_ROW_WAVES ? BW_PSIDE : 13;
+  constexpr int WIN_PER = RW == BW_ROW_WAVES ? BW_WIN_PER : 11;
+  constexpr int WIN_BYTES = RW * WIN_PER * 1024;
+  static_assert(WIN_BYTES >= WROWS * BW_PSIDE * BW_ROW_BYTES, "window covers the rows");
   // Separate arrays, each addressed at compile time, so the compiler never
   // makes a fragment read wait for DMA into another buffer. The weight
   // buffers are declared first so that they sit in the low 64 KB, where
@@ -738,25 +835,35 @@ __global__ __launch_bounds__(128 * BW_ROW_WAVES, 1) void convBoardWindowKernel(c
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   float* stage = OWN_STAGE ? stageArr + wave * 32 * CONV_STAGE_LD : (float*)(win0 + wave * STAGE_BYTES);
-  const int wm = wave % RW;  // row block of WT rows
-  const int wn = wave / RW;  // column half
-  const int loader = wm;
+  const int wm = wave % CW;  // row block of WT rows
+  const int wn = wave / CW;  // column half
+  const int loader = wave % RW;
   const bool loadsWeights = wave < RW;
-  const bool loadsWindow = wave >= RW;
-  int board, colTile;
-  rowColTile(cout / BN, board, colTile);
+  const bool loadsWindow = wave >= RW && wave < 2 * RW;
+  int rowTile, colTile;
+  rowColTile(cout / BN, rowTile, colTile);
+  const int board = RW == BW_ROW_WAVES ? rowTile : rowTile >> 1;
+  // First of this workgroup's rows in the board, and the padded row at
+  // which its window starts (one above the first row's board row).
+  const int rowBase = RW == BW_ROW_WAVES ? 0 : (rowTile & 1) * 96 * RW;
+  const int py0 = rowBase / BW_SIDE;
   const int m0 = board * BW_HW;
   const int mEnd = m0 + BW_HW;
   const int n0 = colTile * BN;
   const int laneRow = lane & 31;
   const int kq = lane >> 5;
   const int cChunks = cinPad / 32;
-  const int steps = 9 * cChunks;
+  // This workgroup's chunks [cBegin, cEnd): all of them, or split
+  // blockIdx.y's share (the host makes every split non-empty).
+  const int perSplit = SPLIT ? (cChunks + (int)gridDim.y - 1) / (int)gridDim.y : cChunks;
+  const int cBegin = SPLIT ? (int)blockIdx.y * perSplit : 0;
+  const int cEnd = SPLIT ? min(cChunks, cBegin + perSplit) : cChunks;
+  const int steps = 9 * cEnd;
   const int tapStride = cout * cinPad;
 
   // Window load i of this wave fills LDS bytes [1024 j, 1024 j + 1024),
   // j = wave + RW i: lane l writes slot q = 64 j + l, which is 16-byte group
-  // q % 5 of window position q / 5 (padded row q / 5 / 21). Element
+  // q % 5 of window position q / 5 (padded row py0 + q / 5 / 21). Element
   // offsets into x are 32-bit: the host keeps tensors below 2^31 elements.
   const half_t* winPtr[WIN_PER];
 #pragma unroll
@@ -765,9 +872,10 @@ __global__ __launch_bounds__(128 * BW_ROW_WAVES, 1) void convBoardWindowKernel(c
     const int pos = q / 5;
     const int grp = q - 5 * pos;
     const int wy = pos / BW_PSIDE;
+    const int py = py0 + wy;
     const int px = pos - BW_PSIDE * wy;
-    const bool onBoard = grp < 4 && wy >= 1 && wy <= BW_SIDE && px >= 1 && px <= BW_SIDE;
-    winPtr[i] = onBoard ? x + ((m0 + (wy - 1) * BW_SIDE + (px - 1)) * cinStride + grp * 8) : kZeroChannels;
+    const bool onBoard = grp < 4 && wy < WROWS && py >= 1 && py <= BW_SIDE && px >= 1 && px <= BW_SIDE;
+    winPtr[i] = onBoard ? x + ((m0 + (py - 1) * BW_SIDE + (px - 1)) * cinStride + grp * 8) : kZeroChannels;
   }
   auto loadWindow = [&](unsigned char* dst, int c, int i) {
     __builtin_amdgcn_global_load_lds((const void*)(winPtr[i] + c * 32), (lds_void_t*)(dst + (loader + RW * i) * 1024), 16, 0, 0);
@@ -799,8 +907,8 @@ __global__ __launch_bounds__(128 * BW_ROW_WAVES, 1) void convBoardWindowKernel(c
   int aBase[RB];
 #pragma unroll
   for(int rb = 0; rb < RB; rb++) {
-    const int i = wm * WT + rb * 32 + laneRow;
-    const int pos = i < BW_HW ? (i / BW_SIDE + 1) * BW_PSIDE + (i % BW_SIDE + 1) : BW_PSIDE + 1;
+    const int i = rowBase + wm * WT + rb * 32 + laneRow;
+    const int pos = i < BW_HW ? (i / BW_SIDE + 1 - py0) * BW_PSIDE + (i % BW_SIDE + 1) : BW_PSIDE + 1;
     aBase[rb] = (pos - BW_PSIDE - 1) * BW_ROW_BYTES + kq * 16;
   }
   // Weight fragment of column block cb, half step ks: the swizzle term of
@@ -815,8 +923,8 @@ __global__ __launch_bounds__(128 * BW_ROW_WAVES, 1) void convBoardWindowKernel(c
   // prologue DMA first, with the stage in win1, measured 2.4 us slower on
   // C2's residual convs.)
   floatx16 acc[RB][CB];
-  if(epi.residual != nullptr) {
-    residualToAcc<half_t, RB, CB, 1>(acc, epi.residual, epi.ldRes, m0 + wm * WT, n0 + wn * WTN, mEnd, stage);
+  if(!SPLIT && epi.residual != nullptr) {
+    residualToAcc<half_t, RB, CB, 1>(acc, epi.residual, epi.ldRes, m0 + rowBase + wm * WT, n0 + wn * WTN, mEnd, stage);
     __syncthreads();
   }
   else {
@@ -830,11 +938,11 @@ __global__ __launch_bounds__(128 * BW_ROW_WAVES, 1) void convBoardWindowKernel(c
   // Prologue: weights of the first LA steps and the window of the first chunk.
   if(loadsWeights) {
 #pragma unroll
-    for(int i = 0; i < LA; i++) loadWeights(wtBuf(i), i);
+    for(int i = 0; i < LA; i++) loadWeights(wtBuf(i), 9 * cBegin + i);
   }
   if(loadsWindow) {
 #pragma unroll
-    for(int i = 0; i < WIN_PER; i++) loadWindow(win0, 0, i);
+    for(int i = 0; i < WIN_PER; i++) loadWindow(win0, cBegin, i);
   }
   waitVmcnt<0>();
   barrierNoFence();
@@ -870,7 +978,7 @@ __global__ __launch_bounds__(128 * BW_ROW_WAVES, 1) void convBoardWindowKernel(c
     unsigned char* nxt = WP ? win0 : win1;
     // The last chunk re-loads itself into the idle window (never read), so
     // every step issues the same loads.
-    const int cNext = c + 1 < cChunks ? c + 1 : c;
+    const int cNext = c + 1 < cEnd ? c + 1 : c;
 #pragma unroll
     for(int t = 0; t < 9; t++) {
       const unsigned char* wCur = wtBuf(P + t);
@@ -914,14 +1022,46 @@ __global__ __launch_bounds__(128 * BW_ROW_WAVES, 1) void convBoardWindowKernel(c
       }
     }
   };
-  for(int c = 0; c < cChunks; c += 2) {
+  // Buffer phase and window parity follow the chunk's position in this
+  // workgroup's range, so a split may start at any chunk.
+  for(int c = cBegin; c < cEnd; c += 2) {
     chunk(std::integral_constant<int, 0>(), std::integral_constant<int, 0>(), c);
-    if(c + 1 < cChunks) chunk(std::integral_constant<int, 9 % NB>(), std::integral_constant<int, 1>(), c + 1);
+    if(c + 1 < cEnd) chunk(std::integral_constant<int, 9 % NB>(), std::integral_constant<int, 1>(), c + 1);
   }
   waitVmcnt<0>();
   __syncthreads();
 
-  storeWaveEpilogue<half_t, RB, CB, true, false>(acc, stage, m0 + wm * WT, n0 + wn * WTN, mEnd, BW_HW, epi);
+  if constexpr(SPLIT) {
+    // Partial sums in the matrix-core C layout: per register, 32 lanes store
+    // 32 consecutive columns of one row.
+    const size_t M = (size_t)batch * BW_HW;
+    float* dst = work + (size_t)blockIdx.y * M * cout;
+#pragma unroll
+    for(int rb = 0; rb < RB; rb++)
+#pragma unroll
+      for(int r = 0; r < 16; r++) {
+        const int i = rowBase + wm * WT + rb * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+        if(i < BW_HW) {
+#pragma unroll
+          for(int cb = 0; cb < CB; cb++) dst[(size_t)(m0 + i) * cout + n0 + wn * WTN + cb * 32 + laneRow] = acc[rb][cb][r];
+        }
+      }
+  }
+  else {
+    storeWaveEpilogue<half_t, RB, CB, true, false>(acc, stage, m0 + rowBase + wm * WT, n0 + wn * WTN, mEnd, BW_HW, epi);
+  }
+}
+
+
+
+template<int ACT>
+__global__ __launch_bounds__(256) void splitKEpilogueKernel(const float* __restrict__ work, int splits, int M, int HW, int cout,
+                                                            ConvEpilogue<half_t> epi) {
+  const int groups = cout / 8;
+  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+  if(idx >= (long)M * groups) return;
+  const int m = (int)(idx / groups);
+  splitKEpilogue8<ACT>(work, splits, M, HW, cout, epi, m, (int)(idx - (long)m * groups) * 8);
 }
 
 // ---------------------------------------------------------------------------
@@ -1343,7 +1483,7 @@ void launchBoardWindow(const half_t* x, int cinStride, int cinPad, int cout, con
   kgh::g_lastConvKernel = name.c_str();
   dim3 grid(g.batch * (cout / BN));
   hipLaunchKernelGGL((convBoardWindowKernel<BN, BN == 64 ? 9 : 6>), grid, dim3(128 * BW_ROW_WAVES), 0, stream, x, cinStride, cinPad,
-                     cout, w, epi);
+                     cout, w, g.batch, epi);
   KGH_CHECK_LAUNCH();
 }
 
@@ -1354,6 +1494,14 @@ bool boardWindowFits(int cinStride, int cinPad, int cout, int bn, BoardGeom g, c
   const long M = (long)g.batch * g.H * g.W;
   return g.H == BW_SIDE && g.W == BW_SIDE && cinPad % 32 == 0 && cinPad <= BW_MAX_CIN && cinStride % 8 == 0 &&
          !epi.maskResidualAdd && !epi.glu && cout % bn == 0 && M * cinStride < (1L << 31) && 9L * cout * cinPad < (1L << 31);
+}
+
+// Split-K at small batches: 64-column tiles, one workgroup per (half board,
+// column tile, split); a split takes one or more whole 32-channel chunks.
+int splitKCount(int cinPad) {
+  const int chunks = cinPad / 32;
+  const int perSplit = (chunks + SPLITK_MAX_SPLITS - 1) / SPLITK_MAX_SPLITS;
+  return (chunks + perSplit - 1) / perSplit;
 }
 
 // Shape conditions of the window kernel apart from batch size.
@@ -1717,6 +1865,40 @@ void launchConv(const T* x, int cinStride, int cin, int cinPad, int cout, int ky
   kgh::g_lastConvKernel = std::is_same<T, half_t>::value ? "convDirectKernel<fp16>" : "convDirectKernel<fp32>";
   hipLaunchKernelGGL(convDirectKernel<T>, dim3((unsigned)blocks), dim3(threads), 0, stream, x, cinStride, cin, cout, ky, kx,
                      wDirect, g, epi);
+  KGH_CHECK_LAUNCH();
+}
+
+bool convSplitKApplies(int cinStride, int cinPad, int cout, int ky, int kx, const void* wPrepared, BoardGeom g,
+                       const ConvEpilogue<half_t>& epi) {
+  // Up to 384 input channels the streamed default kernel is faster, one launch
+  // for two (192 -> 192 at one board: 6.7 us, split-K 6.2 and 4.7 for the
+  // sums); its chain of K steps grows with the channels, split-K's does not.
+  return ky == 3 && kx == 3 && cinPad > 384 && epi.sumSqOut == nullptr && epi.rowNormIn == nullptr && epi.ropeEnd == 0 &&
+         mfmaPathOk<half_t>(cinStride, cinPad, cout, ky, kx, wPrepared, epi) &&
+         boardWindowFits(cinStride, cinPad, cout, SPLITK_BN, g, epi) && cout % 8 == 0;
+}
+
+size_t convSplitKWorkFloats(int cinPad, int cout, BoardGeom g) {
+  return (size_t)splitKCount(cinPad) * g.batch * g.H * g.W * cout;
+}
+
+void launchConvSplitK(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
+                      const ConvEpilogue<half_t>& epi, float* work, hipStream_t stream) {
+  if(!convSplitKApplies(cinStride, cinPad, cout, 3, 3, w, g, epi)) throw KghError(5, "conv: split-K does not apply to this shape");
+  const int splits = splitKCount(cinPad);
+  // Half boards with 32-row wave tiles: at one board, 2 x 3 x 6 = 36
+  // workgroups of 12 waves for a 192-channel conv.
+  kgh::g_lastConvKernel = "convBoardWindowKernel<3x3 fp16, split-K, half a board per workgroup> + splitKEpilogueKernel";
+  hipLaunchKernelGGL((convBoardWindowKernel<SPLITK_BN, 9, true, 2, 32>), dim3(g.batch * 2 * (cout / SPLITK_BN), splits), dim3(128 * 2 * 3),
+                     0, stream, x, cinStride, cinPad, cout, w, g.batch, epi, work);
+  KGH_CHECK_LAUNCH();
+  const int M = g.batch * g.H * g.W;
+  const long threads = (long)M * (cout / 8);
+  const dim3 grid((unsigned)((threads + 255) / 256));
+  withActKind(epi.actKind, epi.outAct != nullptr, [&](auto actTag) {
+    hipLaunchKernelGGL((splitKEpilogueKernel<decltype(actTag)::value>), grid, dim3(256), 0, stream, work, splits, M, g.H * g.W, cout,
+                       epi);
+  });
   KGH_CHECK_LAUNCH();
 }
 

@@ -321,7 +321,7 @@ struct ComputeContext {
   // openCLTunerFile is the model): tables live in <home data dir>/hiptuning.
   bool autoTune = true;
   // hipLowLatency: handles of at most KGH_LOW_LATENCY_MAX_BATCH rows run the
-  // low-latency mode (kgh_handle_set_low_latency), for batch-1 searches.
+  // split-K 3x3 convs (kgh_handle_set_low_latency), for batch-1 searches.
   bool lowLatency = false;
   // hipDebugIntermediateValues: every batch writes the per-block trunk
   // summary lines (kgh_handle_set_layer_dump) to stderr, as a build with
@@ -576,7 +576,7 @@ ComputeHandle* NeuralNet::createComputeHandle(ComputeContext* context, const Loa
                   " useNHWC = true");
     logger->write(prefix + "Model name: " + desc.name + " (" + desc.getShortInfoString() + ")");
     if(context->lowLatency)
-      logger->write(prefix + (lowLatency ? "Low-latency mode enabled"
+      logger->write(prefix + (lowLatency ? "Low-latency (split-K) 3x3 convolutions enabled"
                                          : "hipLowLatency ignored: nnMaxBatchSize above " +
                                              Global::intToString(KGH_LOW_LATENCY_MAX_BATCH)));
   }

@@ -174,7 +174,7 @@ class ComputeContext:
     auto_tune: None keeps the backend default (on), True/False sets
     hipAutoTune; home_data_dir is homeDataDirOverride (tuning tables under
     <dir>/hiptuning); tuner_file sets hipTunerFile; low_latency sets
-    hipLowLatency (handles of max_batch <= 16, see kgh_handle_set_low_latency)."""
+    hipLowLatency (split-K 3x3 convs for handles of max_batch <= 16)."""
 
     def __init__(self, model: LoadedModel, nn_x: int = 19, nn_y: int = 19, use_fp16=None, auto_tune=None,
                  home_data_dir: str = "", tuner_file: str = "", low_latency=None):
@@ -582,7 +582,7 @@ class DeviceHandle:
         hip_check(hip_library().kgh_handle_set_graphs(self._ptr, int(on)))
 
     def set_low_latency(self, on: bool):
-        """kgh_handle_set_low_latency (max_batch <= 16)."""
+        """kgh_handle_set_low_latency: split-K 3x3 convs (max_batch <= 16)."""
         lib = hip_library()
         lib.kgh_handle_set_low_latency.argtypes = [ctypes.c_void_p, ctypes.c_int32]
         hip_check(lib.kgh_handle_set_low_latency(self._ptr, int(on)))
