@@ -209,7 +209,7 @@ __global__ void ropeKernel(T* __restrict__ qkv, int ld, int H, int KV, int dq, c
 // by 16 bytes) and V (transposed, [dim][key], rows padded by 8 bytes) of the
 // item's kv head are staged in LDS once, so each wave then streams the keys
 // from LDS with no further barrier, while the next item's K and V rows load
-// into registers. Wave w owns queries 32w .. 32w+31 and, per block of 32
+// into registers. Each wave owns 32 queries and, per block of 32
 // keys, computes S^T = K Q^T (lane = query, 16 keys per lane), an online
 // softmax per lane, and O^T += V^T P^T with P taken straight from the
 // accumulator registers: the key order inside the second product's k slots
@@ -217,6 +217,13 @@ __global__ void ropeKernel(T* __restrict__ qkv, int ld, int H, int KV, int dq, c
 // of each 16-key step), and V^T is read in that same order. The score products of the next key
 // block are issued before the softmax of the current one, so the matrix
 // cores run them while the vector units work through the softmax.
+// gridDim.y workgroups share an item where there are few: each stages all its
+// keys and takes wavesPerPart of the query waves. A wave's key loop is bound
+// by the vector units, which three waves per SIMD share at 19x19 on one CU.
+// us per launch, six heads of 64, four boards of 19x19: one workgroup per item
+// 16.7, three 12.2 (staging, a round trip to memory, is most of the rest).
+// A test per wave beside q0 costs the 64-dim kernel 132 bytes of scratch per
+// lane (128 boards 4% slower), so a wave without queries has q0 = HW.
 constexpr int FA_THREADS = 768;
 constexpr int FA_MAX_KEYS = 384;
 
@@ -229,7 +236,7 @@ __global__ __launch_bounds__(FA_THREADS, 1) void flashAttentionKernel(const half
                                                                      int KV, const float* __restrict__ mask, int HW,
                                                                      half_t* __restrict__ out, int ldOut, float scale,
                                                                      const float* __restrict__ cosT, const float* __restrict__ sinT,
-                                                                     int learnable, int items) {
+                                                                     int learnable, int items, int wavesPerPart) {
   static_assert(DQ % 16 == 0 && DV % 16 == 0 && DQ <= 64 && DV <= 64, "head dims (LDS holds all keys)");
   constexpr int DVP = (DV + 31) / 32 * 32;
   constexpr int KLD = DQ + 8;             // halves per K row (16-byte pad)
@@ -242,7 +249,7 @@ __global__ __launch_bounds__(FA_THREADS, 1) void flashAttentionKernel(const half
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;
-  const int q0 = wave * 32;
+  const int q0 = wave < wavesPerPart ? ((int)blockIdx.y * wavesPerPart + wave) * 32 : HW;  // HW: no queries
   const int laneRow = lane & 31;
   const int kq = lane >> 5;
   const int qi = q0 + laneRow;
@@ -513,7 +520,7 @@ __global__ __launch_bounds__(FA_THREADS, 1) void flashAttentionKernel(const half
 // halves holds keys k(r) and k(r) + 4, which is one K = 2 step of the second
 // product when V is read at those two keys.
 // Bound: the matrix cores (64 cycles per 32x32x2 step; 4096 cycles per 32x32
-// tile of scores at dims 64/64). Eight boards of 19x19, six heads of 64: 42 us
+// tile of scores at dims 64/64). Eight boards of 19x19, six heads of 64: 37 us
 // per launch against 7.70 ms on one thread per query (whose 128 output
 // accumulators live in scratch memory).
 constexpr int AF_THREADS = 256;
@@ -760,8 +767,12 @@ bool launchFlash(const half_t* qkv, int ld, int kOff, int vOff, int H, int KV, c
   constexpr int perCU = std::max(1, 163840 / ldsBytes);
   const int items = batch * H;
   const int grid = std::min(items, perCU * deviceComputeUnits());
-  hipLaunchKernelGGL((flashAttentionKernel<DQ, DV>), dim3(grid), dim3(FA_THREADS), 0, stream, qkv, ld, kOff, vOff, H, KV, mask, HW,
-                     out, ldOut, scale, cosT, sinT, learnable ? 1 : 0, items);
+  // As many parts as leave each a wave per SIMD and all of them a CU.
+  const int queryWaves = (HW + 31) / 32;
+  const int parts = std::max(std::min((queryWaves + 3) / 4, deviceComputeUnits() / std::max(items, 1)), 1);
+  const int wavesPerPart = (queryWaves + parts - 1) / parts;
+  hipLaunchKernelGGL((flashAttentionKernel<DQ, DV>), dim3(grid, parts), dim3(FA_THREADS), 0, stream, qkv, ld, kOff, vOff, H, KV, mask, HW,
+                     out, ldOut, scale, cosT, sinT, learnable ? 1 : 0, items, wavesPerPart);
   KGH_CHECK_LAUNCH();
   return true;
 }
