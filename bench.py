@@ -194,7 +194,7 @@ def latency(h, call, lm, cfg, batch=1, steps=200):
     out = {"hbm_resident_ms": {"p50": q(lat, 50), "p90": q(lat, 90), "min": q(lat, 0)},
            "pcie_inclusive_ms": host_path(False)}
     if cfg.fp16 and batch <= 16:
-        # The same with hipLowLatency: device-resident
+        # The same with hipLowLatency (3x3 convs in splits of K): device-resident
         # inputs on a one-row device handle, and the host-memory path.
         h.set_low_latency(True)
         for _ in range(5):
@@ -209,7 +209,8 @@ def latency(h, call, lm, cfg, batch=1, steps=200):
         h.set_low_latency(False)
         out["low_latency"] = {"hbm_resident_ms": {"p50": q(fast, 50), "p90": q(fast, 90), "min": q(fast, 0)},
                               "pcie_inclusive_ms": host_path(True),
-                              "what": "hipLowLatency (the default kernels)"}
+                              "what": "hipLowLatency: 3x3 convolutions in up to eight splits of K, fp32 sums added in a "
+                                      "fixed order"}
     out.update({"forwards": steps, "what": "one board per forward, host wall clock from launch to synchronize"})
     return out
 

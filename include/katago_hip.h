@@ -254,12 +254,12 @@ int kgh_handle_set_tuning(kgh_handle* handle, const char* table);
 int kgh_handle_get_tuning(kgh_handle* handle, char* buf, int32_t buflen);
 
 /* Low-latency mode for small batches (config key hipLowLatency of the
- * NeuralNet backend; no counterpart in nninterface.h): every fp16 3x3 conv of
- * more than 384 input channels on 19x19 boards that the one-board kernel takes
- * runs split-K (below that the default kernels are faster), its 32-channel
- * chunks spread over up to eight workgroups per (board, 64 output channels)
- * whose fp32 partial sums a second kernel adds in a fixed order before the
- * epilogue.
+ * NeuralNet backend; no counterpart in nninterface.h): every fp16 3x3 conv
+ * on 19x19 boards that the one-board kernel takes, of 64 input channels and
+ * more, cuts its 32-channel chunks into up to eight splits whose fp32 sums are
+ * added in a fixed order before the epilogue: in the registers of one kernel
+ * up to 704 channels, by a second kernel above. Programs that use the mode keep
+ * their outputs; the default kernels are now as fast or faster.
  * Results are deterministic and independent of the batch size within the
  * mode, but not bitwise equal to the default kernels (other summation order;
  * both stay within the fp16 tolerances of the oracle). Only for handles of

@@ -363,12 +363,12 @@ bool convRopeOk(int cinStride, int cinPad, int cout, int ky, int kx, const void*
 template<typename T>
 bool convNormFoldOk(int cinStride, int cinPad, int cout, int ky, int kx, const void* wPrepared, const ConvEpilogue<T>& epi);
 
-// Split-K form of the one-board 3x3 kernel for small batches (the handle's
-// low-latency mode): the conv's 32-channel chunks are spread over up to eight
-// workgroups per (board, 64-column tile), whose fp32 partial sums
-// (convSplitKWorkFloats floats of work) a second kernel adds in a fixed order
-// before applying the epilogue. Deterministic, but not bitwise equal to the
-// other kernels (different summation order).
+// 3x3 fp16 convs of the handle's low-latency mode: the 32-channel chunks are
+// cut into up to eight splits, whose fp32 sums are added in a fixed order
+// before the epilogue, in the registers of the streamed kernel or, above 704
+// channels, by a second kernel from work (convSplitKWorkFloats floats), the
+// splits being workgroups of the one-board kernel. Deterministic, but not
+// bitwise equal to the default kernels (different summation order).
 bool convSplitKApplies(int cinStride, int cinPad, int cout, int ky, int kx, const void* wPrepared, BoardGeom g,
                        const ConvEpilogue<half_t>& epi);
 size_t convSplitKWorkFloats(int cinPad, int cout, BoardGeom g);

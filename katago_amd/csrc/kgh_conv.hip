@@ -1496,13 +1496,10 @@ bool boardWindowFits(int cinStride, int cinPad, int cout, int bn, BoardGeom g, c
          !epi.maskResidualAdd && !epi.glu && cout % bn == 0 && M * cinStride < (1L << 31) && 9L * cout * cinPad < (1L << 31);
 }
 
-// Split-K at small batches: 64-column tiles, one workgroup per (half board,
-// column tile, split); a split takes one or more whole 32-channel chunks.
-int splitKCount(int cinPad) {
-  const int chunks = cinPad / 32;
-  const int perSplit = (chunks + SPLITK_MAX_SPLITS - 1) / SPLITK_MAX_SPLITS;
-  return (chunks + perSplit - 1) / perSplit;
-}
+// The low-latency mode's sums: a split takes one or more whole 32-channel
+// chunks.
+int splitKChunks(int cinPad) { return (cinPad / 32 + SPLITK_MAX_SPLITS - 1) / SPLITK_MAX_SPLITS; }
+int splitKCount(int cinPad) { return (cinPad / 32 + splitKChunks(cinPad) - 1) / splitKChunks(cinPad); }
 
 // Shape conditions of the window kernel apart from batch size.
 bool tapWindowFits(int cinStride, int cinPad, int cout, int bn, BoardGeom g, const ConvEpilogue<half_t>& epi) {
@@ -1870,10 +1867,7 @@ void launchConv(const T* x, int cinStride, int cin, int cinPad, int cout, int ky
 
 bool convSplitKApplies(int cinStride, int cinPad, int cout, int ky, int kx, const void* wPrepared, BoardGeom g,
                        const ConvEpilogue<half_t>& epi) {
-  // Up to 384 input channels the streamed default kernel is faster, one launch
-  // for two (192 -> 192 at one board: 6.7 us, split-K 6.2 and 4.7 for the
-  // sums); its chain of K steps grows with the channels, split-K's does not.
-  return ky == 3 && kx == 3 && cinPad > 384 && epi.sumSqOut == nullptr && epi.rowNormIn == nullptr && epi.ropeEnd == 0 &&
+  return ky == 3 && kx == 3 && cinPad >= 64 && epi.sumSqOut == nullptr && epi.rowNormIn == nullptr && epi.ropeEnd == 0 &&
          mfmaPathOk<half_t>(cinStride, cinPad, cout, ky, kx, wPrepared, epi) &&
          boardWindowFits(cinStride, cinPad, cout, SPLITK_BN, g, epi) && cout % 8 == 0;
 }
@@ -1885,6 +1879,17 @@ size_t convSplitKWorkFloats(int cinPad, int cout, BoardGeom g) {
 void launchConvSplitK(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
                       const ConvEpilogue<half_t>& epi, float* work, hipStream_t stream) {
   if(!convSplitKApplies(cinStride, cinPad, cout, 3, 3, w, g, epi)) throw KghError(5, "conv: split-K does not apply to this shape");
+  // The streamed kernel adds the splits' sums in registers, the same sums in
+  // the same order as split-K workgroups and a second launch, wherever its
+  // 64-row tile fits the LDS (up to 704 channels). us per forward of four
+  // blocks, in registers / split-K: 448 channels 158 / 169 at one board, 367 /
+  // 465 at 16; 640: 191 / 197, 624 / 698; 704: 202 / 195, 688 / 819; 768, with
+  // 32-row tiles one to a CU: 214 / 209, 1229 / 959. (b18c384nbt at one board:
+  // 836 / 1055 before the streamed kernels.)
+  if(kgh::streamFits(CONV_STREAM3_64, cinStride, cinPad, cout, g, epi)) {
+    kgh::launchStreamParts(x, cinStride, cinPad, cout, w, g, epi, splitKChunks(cinPad), stream);
+    return;
+  }
   const int splits = splitKCount(cinPad);
   // Half boards with 32-row wave tiles: at one board, 2 x 3 x 6 = 36
   // workgroups of 12 waves for a 192-channel conv.

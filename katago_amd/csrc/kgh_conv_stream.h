@@ -19,6 +19,11 @@ bool streamFits(int variant, int cinStride, int cinPad, int cout, BoardGeom g, c
 void launchStream(int variant, const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
                   const ConvEpilogue<half_t>& epi, hipStream_t stream);
 
+// 3x3 with partial sums of partChunks 32-channel chunks each, added in order
+// (the low-latency mode), for shapes that CONV_STREAM3_64 takes.
+void launchStreamParts(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g, const ConvEpilogue<half_t>& epi,
+                       int partChunks, hipStream_t stream);
+
 // fp32 weights (oc, ic, y, x) to the streamed kernels' fragment layout.
 void prepareFragWeights(const float* dW, half_t* dOut, int cout, int cin, int cinPad, int ks, hipStream_t stream);
 

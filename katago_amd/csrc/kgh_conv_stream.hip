@@ -61,10 +61,11 @@ struct StreamDims {
 
 // The plain form of the epilogue (raw and activated outputs, per-board bias):
 // four lanes take the 64 bytes of a row's 32-column block, so every store
-// instruction writes whole 64-byte runs.
-template<int RB, int CB, int ACT>
+// instruction writes whole 64-byte runs. ADD_RES adds a residual that the lane
+// holds in the same places.
+template<int RB, int CB, int ACT, bool ADD_RES>
 __device__ __forceinline__ void storeWaveRows(floatx16 (&acc)[RB][CB], float* stage, int mBase, int nBase, int M, int HW,
-                                              const ConvEpilogue<half_t>& epi) {
+                                              const ConvEpilogue<half_t>& epi, const half8_t (&res)[RB][CB][2]) {
   const int lane = threadIdx.x & 63;
   const int laneRow = lane & 31;
   const int q = lane & 3;       // which 8 of the 32 columns
@@ -113,6 +114,10 @@ __device__ __forceinline__ void storeWaveRows(floatx16 (&acc)[RB][CB], float* st
 #pragma unroll
             for(int j = 0; j < 8; j++) v[p][j] += nb[j];
           }
+          if(ADD_RES && epi.residual != nullptr) {
+#pragma unroll
+            for(int j = 0; j < 8; j++) v[p][j] = (float)res[rb][cb][p][j] + v[p][j];
+          }
           if(rawCols) {
             half8_t o;
 #pragma unroll
@@ -131,10 +136,16 @@ __device__ __forceinline__ void storeWaveRows(floatx16 (&acc)[RB][CB], float* st
   }
 }
 
-template<int KS, int RB, int CB, int WM, int WN, int DEPTH, bool GLU>
+// PARTS (3x3, low-latency mode): every partChunks 32-channel chunks have a sum
+// of their own, started at zero; the sums are added in order, then the bias
+// and the residual. Additions after each part wait for the matrix core, ~1 us
+// of a launch of 7.6 us at 192 channels and one board; a second set of
+// accumulators, added and cleared during the next part's instructions, was
+// slower (the forward 861 us against 836).
+template<int KS, int RB, int CB, int WM, int WN, int DEPTH, bool GLU, bool PARTS>
 __global__ __launch_bounds__(64 * WM * WN, 1) void convStreamKernel(const half_t* __restrict__ x, int cinStride, int cinPad, int cout,
                                                                     const half_t* __restrict__ wf, BoardGeom g, StreamDims sd,
-                                                                    ConvEpilogue<half_t> epi) {
+                                                                    ConvEpilogue<half_t> epi, int partChunks) {
   constexpr int NW = WM * WN;
   constexpr int NT = 64 * NW;
   constexpr int BM = 32 * RB * WM;
@@ -167,12 +178,13 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void convStreamKernel(const half_t
   float* stage = (float*)(win + wave * STREAM_STAGE_BYTES);
   const int winBytes = (winRows * strideB + 1023) / 1024 * 1024;
 
-  // The residual starts the accumulators, so its loads come first: four lanes
-  // per 64-byte row of a 32 x 32 block.
-  const bool resInAcc = epi.residual != nullptr && !epi.maskResidualAdd;
+  // The residual starts the accumulators (or waits for the end), so its loads
+  // come first: four lanes per 64-byte row of a 32 x 32 block.
+  const bool loadRes = epi.residual != nullptr && !epi.maskResidualAdd;
+  const bool resInAcc = !PARTS && loadRes;
   const int quarter = lane & 3, qRow = lane >> 2;
   half8_t res[RB][CB][2];
-  if(resInAcc) {
+  if(loadRes) {
 #pragma unroll
     for(int rb = 0; rb < RB; rb++)
 #pragma unroll
@@ -342,8 +354,28 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void convStreamKernel(const half_t
           });
       }
     };
-    for(int c = 0; c + 1 < chunks; c++) chunk(c, std::integral_constant<bool, false>());
-    chunk(chunks - 1, std::integral_constant<bool, true>());
+    if constexpr(PARTS) {
+      static_assert(RB == 1 && CB == 1, "registers for the sum");
+      floatx16 sum = acc[0][0];
+      int left = partChunks;
+      for(int c = 0; c + 1 < chunks; c++) {
+        chunk(c, std::integral_constant<bool, false>());
+        if(--left == 0) {
+          left = partChunks;
+#pragma unroll
+          for(int r = 0; r < 16; r++) {
+            sum[r] += acc[0][0][r];
+            acc[0][0][r] = 0.0f;
+          }
+        }
+      }
+      chunk(chunks - 1, std::integral_constant<bool, true>());
+      acc[0][0] = sum + acc[0][0];
+    }
+    else {
+      for(int c = 0; c + 1 < chunks; c++) chunk(c, std::integral_constant<bool, false>());
+      chunk(chunks - 1, std::integral_constant<bool, true>());
+    }
   }
   else {
     // Two A slots, read one step ahead; reads past the last step repeat it.
@@ -372,9 +404,9 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void convStreamKernel(const half_t
 
   __syncthreads();  // every wave is done with the window before it holds the stages
   if constexpr(!GLU) {
-    if(epi.sumSqOut == nullptr && !rowNorm && epi.ropeEnd == 0 && (resInAcc || epi.residual == nullptr)) {
+    if(epi.sumSqOut == nullptr && !rowNorm && epi.ropeEnd == 0 && (loadRes || epi.residual == nullptr)) {
       withActKind(epi.actKind, epi.outAct != nullptr, [&](auto actTag) {
-        storeWaveRows<RB, CB, decltype(actTag)::value>(acc, stage, mWave, nWave, M, HW, epi);
+        storeWaveRows<RB, CB, decltype(actTag)::value, PARTS>(acc, stage, mWave, nWave, M, HW, epi, res);
       });
       return;
     }
@@ -420,17 +452,17 @@ struct Stream {
            4 * ((M + BM) / BM * (cout / BN)) * (cout / BN) < (1L << 32) &&
            streamLdsBytes<KS, BM, NW>(cinPad, g.W) <= STREAM_MAX_LDS;
   }
-  template<bool GLU>
+  template<bool GLU, bool PARTS>
   static void run(const half_t* x, int cinStride, int cinPad, int cout, const half_t* wf, BoardGeom g, const ConvEpilogue<half_t>& epi,
-                  hipStream_t stream) {
+                  int partChunks, hipStream_t stream) {
     const int M = g.batch * g.H * g.W;
     const int colTiles = cout / BN;
     const dim3 grid((M + BM - 1) / BM * colTiles), block(64 * NW);
     const int lds = streamLdsBytes<KS, BM, NW>(cinPad, g.W);
     const unsigned per = cinPad / 8 + 1;
     const StreamDims sd = {per, divMagic(per), divMagic(g.H * g.W), divMagic(g.W), (unsigned)colTiles, divMagic(colTiles)};
-    hipLaunchKernelGGL((convStreamKernel<KS, RB, CB, WM, WN, DEPTH, GLU>), grid, block, lds, stream, x, cinStride, cinPad, cout, wf, g,
-                       sd, epi);
+    hipLaunchKernelGGL((convStreamKernel<KS, RB, CB, WM, WN, DEPTH, GLU, PARTS>), grid, block, lds, stream, x, cinStride, cinPad, cout,
+                       wf, g, sd, epi, partChunks);
     KGH_CHECK_LAUNCH();
   }
   // w: the prepared weights; the fragment layout follows the first.
@@ -442,11 +474,18 @@ struct Stream {
     const half_t* wf = w + (size_t)KS * KS * cout * cinPad;
     if constexpr(KS == 1) {
       if(epi.glu) {
-        run<true>(x, cinStride, cinPad, cout, wf, g, epi, stream);
+        run<true, false>(x, cinStride, cinPad, cout, wf, g, epi, 0, stream);
         return;
       }
     }
-    run<false>(x, cinStride, cinPad, cout, wf, g, epi, stream);
+    run<false, false>(x, cinStride, cinPad, cout, wf, g, epi, 0, stream);
+  }
+  static void launchParts(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
+                          const ConvEpilogue<half_t>& epi, int partChunks, hipStream_t stream) {
+    static const std::string name = kernelLabel("convStreamKernel<%dx%d fp16, %dx%d tiles, %d waves of %dx%d, partial sums>", KS, KS, BM,
+                                                BN, NW, 32 * RB, 32 * CB);
+    kgh::g_lastConvKernel = name.c_str();
+    run<false, true>(x, cinStride, cinPad, cout, w + (size_t)KS * KS * cout * cinPad, g, epi, partChunks, stream);
   }
 };
 
@@ -500,6 +539,17 @@ int streamTile3x3(int cinStride, int cinPad, int cout, BoardGeom g, const ConvEp
     return CONV_STREAM3_128;
   if(streamFits(CONV_STREAM3_192, cinStride, cinPad, cout, g, epi)) return CONV_STREAM3_192;
   return CONV_AUTO;
+}
+
+// The 32-row tile while its workgroups fit the 256 CUs one to a CU, else 64
+// rows (streamTile3x3 has both tiles' times).
+void launchStreamParts(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g, const ConvEpilogue<half_t>& epi,
+                       int partChunks, hipStream_t stream) {
+  const long M = (long)g.batch * g.H * g.W;
+  if((M + 31) / 32 * (cout / 64) > 256)
+    Stream<3, 1, 1, 2, 2, 9>::launchParts(x, cinStride, cinPad, cout, w, g, epi, partChunks, stream);
+  else
+    Stream<3, 1, 1, 1, 2, 9>::launchParts(x, cinStride, cinPad, cout, w, g, epi, partChunks, stream);
 }
 
 // 1x1: every shape below 24 row tiles of 192 (a few boards: t12d384h6 at four,

@@ -582,7 +582,7 @@ class DeviceHandle:
         hip_check(hip_library().kgh_handle_set_graphs(self._ptr, int(on)))
 
     def set_low_latency(self, on: bool):
-        """kgh_handle_set_low_latency: split-K 3x3 convs (max_batch <= 16)."""
+        """kgh_handle_set_low_latency: 3x3 convs in splits of K (max_batch <= 16)."""
         lib = hip_library()
         lib.kgh_handle_set_low_latency.argtypes = [ctypes.c_void_p, ctypes.c_int32]
         hip_check(lib.kgh_handle_set_low_latency(self._ptr, int(on)))

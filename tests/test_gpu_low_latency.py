@@ -1,13 +1,18 @@
-"""Low-latency mode (hipLowLatency / kgh_handle_set_low_latency): split-K 3x3
-convolutions for handles of at most 16 rows. Checked against the CPU oracle at
-the fp16 whole-net tolerances (the summation order differs from the default
-kernels, so these rows are not bitwise equal to a default handle's), and for
+"""Low-latency mode (hipLowLatency / kgh_handle_set_low_latency): 3x3
+convolutions whose sums are cut into up to eight splits, for handles of at
+most 16 rows. Checked against the CPU oracle at the fp16 whole-net tolerances
+(the summation order differs from the default kernels, so these rows are not
+bitwise equal to a default handle's), against recorded bits, and for
 batch-size independence within the mode."""
+import os
+
 import numpy as np
 import pytest
 
 from katago_amd import modelgen, nn
 from oracle import oracle
+from conftest import GOLDEN
+from golden import make_low_latency_golden as recorded
 from test_gpu_parity import _compare
 
 pytestmark = pytest.mark.gpu
@@ -41,8 +46,8 @@ def test_low_latency_matches_oracle(model_dir, n, board_sizes, cfg_idx):
 
 
 def test_low_latency_rows_do_not_depend_on_batch(model_dir):
-    """Within the mode every call runs the same split-K kernels, so a row's
-    outputs are bitwise the same at batch 1 and inside a batch of 12; the mode
+    """Within the mode every call adds the same splits in the same order, so a
+    row's outputs are bitwise the same at batch 1 and inside a batch of 12; the mode
     is deterministic (a repeat gives the same bits)."""
     cfg = modelgen.configs()[3]
     lm = nn.LoadedModel(modelgen.ensure_model(model_dir, cfg))
@@ -59,8 +64,9 @@ def test_low_latency_rows_do_not_depend_on_batch(model_dir):
 
 
 def test_low_latency_close_to_default_kernels(model_dir):
-    """The split-K sums differ from the default kernels only by fp32 rounding
-    order: the outputs agree far inside the fp16 tolerances."""
+    """The splits' sums differ from the default kernels only by fp32 rounding
+    order: the outputs agree far inside the fp16 tolerances, but are not the
+    same bits."""
     cfg = modelgen.configs()[2]
     lm = nn.LoadedModel(modelgen.ensure_model(model_dir, cfg))
     sp, gl = modelgen.synthetic_inputs(cfg.input_seed, 4)
@@ -71,6 +77,34 @@ def test_low_latency_close_to_default_kernels(model_dir):
     for k in a:
         d = np.abs(a[k] - b[k]).max()
         assert d <= 5e-3, (k, d)
+    assert not np.array_equal(a["policy"], b["policy"])
+
+
+@pytest.mark.parametrize("arch", recorded.NETS, ids=lambda a: a.name)
+def test_low_latency_gives_the_recorded_bits(model_dir, arch):
+    """A row is rounded as it always was in this mode, whichever kernels add
+    the splits: in registers up to 704 channels, split-K workgroups above; at
+    a batch of two and, on the 64-row tiles, of 16."""
+    lm = nn.LoadedModel(recorded.model_file(model_dir, arch))
+    want = np.load(os.path.join(GOLDEN, "low_latency.npz"))
+    ctx = nn.ComputeContext(lm, 19, 19, use_fp16=True, low_latency=True)
+    rows = recorded.inputs()
+    for n in (2, 16):
+        got = nn.ComputeHandle(ctx, max_batch=n).get_output(*(np.concatenate([r] * (n // 2)) for r in rows))
+        for k in got:
+            assert np.array_equal(got[k][:2], want[f"{arch.name}/{k}"]) and np.array_equal(got[k][-2:], got[k][:2]), (n, k)
+
+    dm = nn.DeviceModel(lm, use_fp16=True)
+    h = nn.DeviceHandle(dm, 2)
+    h.set_low_latency(True)
+    h.set_profiling(True)
+    dev = [nn.DeviceBuffer.from_array(r) for r in rows]
+    out = nn.DeviceBuffer(2 * h.row_floats * 4)
+    h.forward_device(2, *(b.ptr for b in dev), out.ptr)
+    h.synchronize()
+    kernels = " ".join(r[4] for r in h.profile_kernels() if r[0] == 0)
+    assert ("split-K" if arch.mid_c > 704 else "partial sums") in kernels, kernels
+    dm.close()
 
 
 def test_low_latency_device_handle_limits(model_dir):
