@@ -264,7 +264,8 @@ int kgh_handle_get_tuning(kgh_handle* handle, char* buf, int32_t buflen);
  * mode, but not bitwise equal to the default kernels (other summation order;
  * both stay within the fp16 tolerances of the oracle). Only for handles of
  * max_batch <= KGH_LOW_LATENCY_MAX_BATCH; enabling allocates the partial-sum
- * buffer (8 * max_batch * nn_x * nn_y * widest channel count floats). */
+ * buffer (8 * max_batch * nn_x * nn_y * widest channel count floats) of nets of
+ * more than 704 channels. */
 #define KGH_LOW_LATENCY_MAX_BATCH 16
 int kgh_handle_set_low_latency(kgh_handle* handle, int32_t enabled);
 

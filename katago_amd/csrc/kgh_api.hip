@@ -589,7 +589,8 @@ struct kgh_handle {
   std::vector<GraphEntry> graphs;
 
   // Low-latency mode (kgh_handle_set_low_latency): the 3x3 convs the split-K
-  // path takes run with their fp32 partial sums in splitWork.
+  // path takes run with their fp32 partial sums in splitWork (null for nets
+  // without convs that need it).
   bool lowLatency = false;
   float* splitWork = nullptr;
 
@@ -2150,11 +2151,13 @@ int kgh_handle_set_low_latency(kgh_handle* handle, int32_t enabled) {
     requireHandle(handle);
     if(enabled && handle->maxBatch > KGH_LOW_LATENCY_MAX_BATCH)
       invalid("low-latency mode takes handles of max_batch <= " + std::to_string(KGH_LOW_LATENCY_MAX_BATCH));
-    if(enabled && handle->splitWork == nullptr) {
-      // Up to eight splits of the widest activation of the net.
-      const Net& net = handle->model->net;
-      int maxC = std::max(net.tmpC, 1);
-      for(int c : net.depthC) maxC = std::max(maxC, c);
+    // Up to eight splits of the widest activation of the net, if any is wide
+    // enough for a split-K conv.
+    const Net& net = handle->model->net;
+    int maxC = std::max(net.tmpC, 1);
+    for(int c : net.depthC) maxC = std::max(maxC, c);
+    maxC = (int)roundUp(maxC, 32);
+    if(enabled && handle->splitWork == nullptr && kgh::convSplitKNeedsWork(maxC, BoardGeom{handle->maxBatch, handle->H, handle->W})) {
       KGH_HIP_CHECK(hipSetDevice(handle->model->device));
       handle->splitWork = handle->arena.allocN<float>((size_t)8 * handle->maxBatch * handle->H * handle->W * maxC);
     }

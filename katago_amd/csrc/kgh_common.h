@@ -366,12 +366,13 @@ bool convNormFoldOk(int cinStride, int cinPad, int cout, int ky, int kx, const v
 // 3x3 fp16 convs of the handle's low-latency mode: the 32-channel chunks are
 // cut into up to eight splits, whose fp32 sums are added in a fixed order
 // before the epilogue, in the registers of the streamed kernel or, above 704
-// channels, by a second kernel from work (convSplitKWorkFloats floats), the
-// splits being workgroups of the one-board kernel. Deterministic, but not
-// bitwise equal to the default kernels (different summation order).
+// channels, by a second kernel from work (8 * M * cout floats), the splits
+// being workgroups of the one-board kernel. Deterministic, but not bitwise
+// equal to the default kernels (different summation order).
 bool convSplitKApplies(int cinStride, int cinPad, int cout, int ky, int kx, const void* wPrepared, BoardGeom g,
                        const ConvEpilogue<half_t>& epi);
-size_t convSplitKWorkFloats(int cinPad, int cout, BoardGeom g);
+// Whether such a conv of cinPad input channels (and any wider one) uses work.
+bool convSplitKNeedsWork(int cinPad, BoardGeom g);
 void launchConvSplitK(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
                       const ConvEpilogue<half_t>& epi, float* work, hipStream_t stream);
 

@@ -1872,8 +1872,9 @@ bool convSplitKApplies(int cinStride, int cinPad, int cout, int ky, int kx, cons
          boardWindowFits(cinStride, cinPad, cout, SPLITK_BN, g, epi) && cout % 8 == 0;
 }
 
-size_t convSplitKWorkFloats(int cinPad, int cout, BoardGeom g) {
-  return (size_t)splitKCount(cinPad) * g.batch * g.H * g.W * cout;
+bool convSplitKNeedsWork(int cinPad, BoardGeom g) {
+  const ConvEpilogue<half_t> plain = {};
+  return !kgh::streamFits(CONV_STREAM3_64, cinPad, cinPad, 64, g, plain);
 }
 
 void launchConvSplitK(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
@@ -1890,6 +1891,7 @@ void launchConvSplitK(const half_t* x, int cinStride, int cinPad, int cout, cons
     kgh::launchStreamParts(x, cinStride, cinPad, cout, w, g, epi, splitKChunks(cinPad), stream);
     return;
   }
+  if(work == nullptr) throw KghError(5, "conv: no split-K work buffer");
   const int splits = splitKCount(cinPad);
   // Half boards with 32-row wave tiles: at one board, 2 x 3 x 6 = 36
   // workgroups of 12 waves for a 192-channel conv.

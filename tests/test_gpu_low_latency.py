@@ -4,6 +4,7 @@ most 16 rows. Checked against the CPU oracle at the fp16 whole-net tolerances
 (the summation order differs from the default kernels, so these rows are not
 bitwise equal to a default handle's), against recorded bits, and for
 batch-size independence within the mode."""
+import ctypes
 import os
 
 import numpy as np
@@ -121,4 +122,25 @@ def test_low_latency_device_handle_limits(model_dir):
     h.set_low_latency(True)
     h.set_low_latency(False)
     h.close()
+    dm.close()
+
+
+@pytest.mark.parametrize("arch,allocates", [(recorded.NETS[2], False), (recorded.NETS[6], True)], ids=["c384-192", "c768"])
+def test_partial_sum_buffer_only_for_nets_that_use_it(model_dir, arch, allocates):
+    """Enabling the mode allocates the split-K partial sums (8 * 16 * 361 *
+    channels floats: 142 MB at 768 channels) only where a conv is too wide to
+    add them in registers."""
+    hip = nn.hip_library()  # its handle finds the runtime it is linked with
+
+    def free():
+        now, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(now), ctypes.byref(total)) == 0
+        return now.value
+
+    dm = nn.DeviceModel(nn.LoadedModel(recorded.model_file(model_dir, arch)), use_fp16=True)
+    h = nn.DeviceHandle(dm, 16)
+    h.synchronize()
+    before = free()
+    h.set_low_latency(True)
+    assert (before - free() > 30e6) == allocates
     dm.close()
