@@ -311,11 +311,11 @@ enum ConvVariant {
   CONV_DMA1H_192,  // 1x1 fp16 DMA kernel with 192-row tiles, two workgroups per CU
   CONV_DMA1H_128,
   CONV_DMA1H_64,
-  CONV_RETIRED_19,
+  CONV_BOARD_HALF_64,  // the one-board kernel on half a board per workgroup (two per CU), 64 output channels per tile
   CONV_RETIRED_20,
   CONV_ALLK1_32,  // 1x1 fp16 kernel for small row counts: 64-row tiles, every input channel in LDS at once
   CONV_DMA1_256_GLU,  // 1x1 fp16 DMA kernel, 384 x 256 tiles, gated (SwiGLU) epilogue only
-  CONV_RETIRED_23,
+  CONV_BOARD_HALF_64_T32,  // the half-board kernel with 32-row wave tiles (12 waves per workgroup)
   CONV_RETIRED_24,
   CONV_STREAM3_32,  // 3x3 fp16 streamed-weight kernel (any board size), 32 rows x 64 output channels per tile
   CONV_STREAM3_64,

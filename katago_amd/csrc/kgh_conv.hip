@@ -23,6 +23,7 @@
 #include <string>
 #include <type_traits>
 #include <cstdint>
+#include <utility>
 #include <vector>
 
 namespace kgh {
@@ -1475,15 +1476,15 @@ void launchTapWindow(const half_t* x, int cinStride, int cinPad, int cout, const
   KGH_CHECK_LAUNCH();
 }
 
-template<int BN>
+template<int BN, int RW = BW_ROW_WAVES, int WT = BW_WTM>
 void launchBoardWindow(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
                        const ConvEpilogue<half_t>& epi, hipStream_t stream) {
-  static const std::string name = kernelLabel("convBoardWindowKernel<3x3 fp16, BN=%d, one board per workgroup, %d-row wave tiles>",
-                                              BN, BW_WTM);
+  static const std::string name = kernelLabel("convBoardWindowKernel<3x3 fp16, BN=%d, %s, %d-row wave tiles>", BN,
+                                              RW == BW_ROW_WAVES ? "one board per workgroup" : "half a board per workgroup", WT);
   kgh::g_lastConvKernel = name.c_str();
-  dim3 grid(g.batch * (cout / BN));
-  hipLaunchKernelGGL((convBoardWindowKernel<BN, BN == 64 ? 9 : 6>), grid, dim3(128 * BW_ROW_WAVES), 0, stream, x, cinStride, cinPad,
-                     cout, w, g.batch, epi);
+  dim3 grid(g.batch * (RW == BW_ROW_WAVES ? 1 : 2) * (cout / BN));
+  hipLaunchKernelGGL((convBoardWindowKernel<BN, BN == 64 ? 9 : 6, false, RW, WT>), grid, dim3(128 * RW * BW_WTM / WT), 0, stream, x,
+                     cinStride, cinPad, cout, w, g.batch, epi);
   KGH_CHECK_LAUNCH();
 }
 
@@ -1508,12 +1509,13 @@ bool tapWindowFits(int cinStride, int cinPad, int cout, int bn, BoardGeom g, con
          cout % bn == 0 && M * cinStride < (1L << 31) && 9L * cout * cinPad < (1L << 31);
 }
 
-// The window kernel: fp16, 3x3, plain residual adds (it starts the
-// accumulators from the residual), boards at most TW_PAD_MAX - 1 wide, enough
-// rows for at least 128 of its 384-row tiles (smaller batches keep more CUs
-// busy with the 128-row kernel), 32-bit element offsets.
-bool dispatchTapWindow(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
-                               const ConvEpilogue<half_t>& epi, hipStream_t stream) {
+// 3x3 fp16 convs with a plain residual add (it starts the accumulators): one
+// board per workgroup, streamed weights, or the tap-window kernel; false where
+// only the 128-row tile kernel takes the shape (other column counts, masked
+// residuals, offsets past 32 bits) or is the fastest. Every kernel gives the
+// same bits.
+bool dispatch3x3(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g, const ConvEpilogue<half_t>& epi,
+                 hipStream_t stream) {
   const long M = (long)g.batch * g.H * g.W;
   // 19x19 boards, one per workgroup with 192- or 128-column tiles, where those
   // fill at least three quarters of their rounds of the 256 CUs: b18c384nbt's
@@ -1529,39 +1531,89 @@ bool dispatchTapWindow(const half_t* x, int cinStride, int cinPad, int cout, con
     else launchBoardWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
     return true;
   }
+  const bool tap = tapWindowFits(cinStride, cinPad, cout, 64, g, epi);
+  const long tapRows = (M + TW_BM - 1) / TW_BM;
+  auto rounds = [](long workgroups) { return (workgroups + 255) / 256; };
   const int tile = kgh::streamTile3x3(cinStride, cinPad, cout, g, epi);
   if(tile != CONV_AUTO) {
-    kgh::launchStream(tile, x, cinStride, cinPad, cout, w, g, epi, stream);
+    // Streamed 192-row tiles run one to a CU (224 to 320 input channels). A
+    // round of whole boards with 64 columns takes 1.9 times as long as one of
+    // theirs (320 channels, us per forward of eight convs: 96 boards, 2 rounds
+    // against 4, 655 and 676; 240 boards, 5 against 9, 1552 and 1474), with 128
+    // columns 2.75 times (256 channels: 80 boards, 1 against 3, 417 and 441; 144
+    // boards, 2 against 5, 822 and 750), a round of the tap-window kernel with
+    // 128 columns 3.45 times (256 channels, 280 boards 18x18, 2 against 8: 1099
+    // and 1201; 200 boards, 2 against 6: 972 and 884).
+    const long streamRounds = tile == CONV_STREAM3_192 ? rounds((M + 191) / 192 * (cout / 64)) : 0;
+    if(board && wide == 64 && 1.9 * rounds(boards) < streamRounds) launchBoardWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else if(board && wide == 128 && 2.75 * rounds(boards) < streamRounds)
+      launchBoardWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else if(!board && tap && wide == 128 && 3.45 * rounds(tapRows * (cout / 128)) < streamRounds)
+      launchTapWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else kgh::launchStream(tile, x, cinStride, cinPad, cout, w, g, epi, stream);
     return true;
   }
   // Too many input channels for two streamed 128-row windows per CU or one of
-  // 192 rows (above about 320), and more than one round of smaller tiles. At
-  // 19x19, one board per workgroup from 128 of its 64-column tiles (384 -> 384
-  // at 40 boards: forwards of six blocks 636 us, 689 on streamed 128-row tiles;
-  // 512 -> 512 at 24: 706, 824 on half boards, 921 on streamed 64-row tiles).
-  // Else the largest streamed tile that fits, and the tap-window kernel where
-  // that is 64 rows and there are 128 of its row tiles (512 channels, 300
-  // boards 13x13: 301 us; at 100 boards 64 streamed rows take 115 us, the
-  // 128-row tile kernel 201).
-  if(board && (long)g.batch * (cout / 64) >= 128) {
-    if(boards >= 160 && wide == 192) launchBoardWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream);
-    else if(boards >= 160 && wide == 128) launchBoardWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
-    else launchBoardWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
+  // 192 rows (above about 320), and more than one round of smaller tiles: the
+  // largest streamed tile that fits, or one of the kernels that stage a chunk
+  // at a time. Figures: us per forward of eight convs.
+  int streamed = CONV_AUTO, rows = 1;
+  for(const auto& t : {std::pair<int, int>{CONV_STREAM3_128, 128}, {CONV_STREAM3_64, 64}, {CONV_STREAM3_32, 32}})
+    if(streamed == CONV_AUTO && kgh::streamFits(t.first, cinStride, cinPad, cout, g, epi)) {
+      streamed = t.first;
+      rows = t.second;
+    }
+  const bool stream128 = streamed == CONV_STREAM3_128;
+  const long streamTiles = streamed == CONV_AUTO ? LONG_MAX : (M + rows - 1) / rows * (cout / 64);
+  if(board && cinPad > 320) {
+    const long whole = (long)g.batch * (cout / 64);  // workgroups of whole boards with 64 columns
+    // Half a round of whole boards or less: half boards with 32-row wave tiles
+    // (384 channels, 16 boards: 268, streamed 128 rows 303; 768, 8 boards: 435
+    // and 699 on 32 rows), but two rounds of streamed 64- or 32-row tiles (512,
+    // 8 boards: 289, half boards 308; 768, 2 boards: 323 and 403).
+    // One round: whole boards, or two rounds of streamed 128-row tiles (384, 24
+    // boards: 320, whole boards 369; 32 boards, three rounds: 441 and 391).
+    // Beyond: 128 columns for one round of their workgroups (768, 40 boards:
+    // 1180, 192 columns 1305), then the widest columns; without them streamed
+    // 128 rows (448, 40 boards: 657, half boards with 96-row wave tiles 719) or
+    // those half boards, to one and a half rounds of whole boards.
+    if(whole <= 128) {
+      if(!stream128 && streamTiles <= 512) kgh::launchStream(streamed, x, cinStride, cinPad, cout, w, g, epi, stream);
+      else launchBoardWindow<64, 2, 32>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    }
+    else if(whole <= 256) {
+      if(stream128 && streamTiles <= 512) kgh::launchStream(streamed, x, cinStride, cinPad, cout, w, g, epi, stream);
+      else launchBoardWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    }
+    else if(wide == 192 && boards >= 160 && (cout % 128 != 0 || whole > 512)) launchBoardWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else if(cout % 128 == 0) launchBoardWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else if(whole > 384) launchBoardWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else if(stream128) kgh::launchStream(streamed, x, cinStride, cinPad, cout, w, g, epi, stream);
+    else launchBoardWindow<64, 2>(x, cinStride, cinPad, cout, w, g, epi, stream);
     return true;
   }
-  for(int v : {CONV_STREAM3_128, CONV_STREAM3_64, CONV_STREAM3_32}) {
-    if(v != CONV_STREAM3_128 && M >= 128L * TW_BM && tapWindowFits(cinStride, cinPad, cout, 64, g, epi)) {
-      if(wide == 192) launchTapWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream);
-      else if(wide == 128) launchTapWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
-      else launchTapWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
-      return true;
-    }
-    if(kgh::streamFits(v, cinStride, cinPad, cout, g, epi)) {
-      kgh::launchStream(v, x, cinStride, cinPad, cout, w, g, epi, stream);
-      return true;
-    }
+  // Other boards: the streamed tile up to a number of rows from which the
+  // tap-window kernel is faster. 128 rows: from 84 of its row tiles where its
+  // columns are wider (384 channels, 150 boards 13x13, 67 tiles: 749 streamed,
+  // 749; 200 boards, 89 tiles: 993 and 905). 64 rows: from 34 (512 channels, 60
+  // boards 13x13: 635 and 770; 80 boards, 36 tiles: 845 and 806). 32 rows: where
+  // they number more than six to a CU (1024 channels, 16 boards 13x13: 1191 and
+  // 1316; 20 boards: 1429 and 1312), and there the tile kernel takes boards too
+  // wide for it. The tap-window kernel has 192 columns where they give 144
+  // workgroups (768 channels, 32 boards 18x18, 108: 1454, 128 columns 1071).
+  const bool tapBest = stream128                       ? wide > 64 && tapRows >= 84
+                       : streamed == CONV_STREAM3_64 ? tapRows >= 34
+                       : streamed == CONV_STREAM3_32 ? streamTiles > 6 * 256
+                                                     : M >= 128L * TW_BM;
+  if(tap && tapBest) {
+    if(wide == 192 && (cout % 128 != 0 || tapRows * (cout / 192) >= 144)) launchTapWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else if(cout % 128 == 0) launchTapWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else launchTapWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    return true;
   }
-  return false;
+  if(streamed == CONV_AUTO || (streamed == CONV_STREAM3_32 && streamTiles > 6 * 256)) return false;
+  kgh::launchStream(streamed, x, cinStride, cinPad, cout, w, g, epi, stream);
+  return true;
 }
 
 // 384 x 256 tiles for gated (SwiGLU) convs only: at 256 columns the
@@ -1661,7 +1713,8 @@ bool variantFits(int v, int ky, int cinStride, int cinPad, int cout, BoardGeom g
     if(v == CONV_TW_64) return tapWindowFits(cinStride, cinPad, cout, 64, g, epi);
     if(v == CONV_BOARD_192) return boardWindowFits(cinStride, cinPad, cout, 192, g, epi);
     if(v == CONV_BOARD_128) return boardWindowFits(cinStride, cinPad, cout, 128, g, epi);
-    if(v == CONV_BOARD_64) return boardWindowFits(cinStride, cinPad, cout, 64, g, epi);
+    if(v == CONV_BOARD_64 || v == CONV_BOARD_HALF_64 || v == CONV_BOARD_HALF_64_T32)
+      return boardWindowFits(cinStride, cinPad, cout, 64, g, epi);
     if(v >= CONV_STREAM3_32 && v <= CONV_STREAM3_192) return kgh::streamFits(v, cinStride, cinPad, cout, g, epi);
   }
   else {
@@ -1705,6 +1758,8 @@ void launchVariant(int v, int ky, const half_t* x, int cinStride, int cinPad, in
     case CONV_BOARD_192: launchBoardWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
     case CONV_BOARD_128: launchBoardWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
     case CONV_BOARD_64: launchBoardWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
+    case CONV_BOARD_HALF_64: launchBoardWindow<64, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
+    case CONV_BOARD_HALF_64_T32: launchBoardWindow<64, 2, 32>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
     case CONV_ALLK1_32: launch1x1AllK(x, cinStride, cinPad, cout, w, g, epi, stream); return;
     case CONV_DMA1_192: launch1x1Dma<192>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
     case CONV_DMA1_128: launch1x1Dma<128>(x, cinStride, cinPad, cout, w, g, epi, stream); return;
@@ -1833,7 +1888,7 @@ void launchConv(const T* x, int cinStride, int cin, int cinPad, int cout, int ky
     }
     else if(mfmaPathOk<T>(cinStride, cinPad, cout, ky, kx, wPrepared, epi)) {
       if(ky == 3 && kx == 3) {
-        done = dispatchTapWindow(x, cinStride, cinPad, cout, (const T*)wPrepared, g, epi, stream);
+        done = dispatch3x3(x, cinStride, cinPad, cout, (const T*)wPrepared, g, epi, stream);
         if(!done) done = dispatchMfmaTile<T, 3>(x, cinStride, cinPad, cout, (const T*)wPrepared, g, epi, stream);
       }
       else if(ky == 1 && kx == 1) {

@@ -28,6 +28,10 @@ def _nbt(t, m):
                          "ACTIVATION_MISH", residual_gain=0.5)
 
 
+def _block(c):
+    return modelgen.Arch("block%d" % c, 15, c, c, 32, ["regular"], 16, 16, 32, 48, "ACTIVATION_RELU", residual_gain=0.5)
+
+
 TRANSFORMER = modelgen.Arch("streamtflrs", 17, 128, 128, 32, ["attention", "ffn"], 16, 16, 32, 48, "ACTIVATION_SILU", heads=2,
                             kv_heads=2, q_head_dim=64, v_head_dim=64, ffn_c=192, learnable_rope=True, trunk_rmsnorm=True)
 
@@ -54,4 +58,47 @@ def test_every_tile_gives_the_tile_kernels_bits(model_dir, arch):
         assert np.isfinite(want).all()
         for v in [0] + STREAM:
             assert np.array_equal(forward(v), want), (n, x, y, v)
+        h.close()
+
+
+# Channels, then (boards, side, what the kernel's name holds) on both sides of
+# the lines that the built-in choice draws for 3x3 convs of 224 channels and more.
+CHOICES = [
+    (256, [(64, 19, "192x64 tiles"), (80, 19, "BN=128, one board"), (200, 13, "192x64 tiles"), (256, 13, "convTapWindowKernel<3x3 fp16, BN=128")]),
+    (320, [(80, 19, "192x64 tiles"), (96, 19, "BN=64, one board")]),
+    (384, [(14, 19, "128x64 tiles"), (16, 19, "half a board per workgroup, 32-row"), (24, 19, "128x64 tiles"), (32, 19, "BN=64, one board"),
+           (48, 19, "BN=128, one board"), (150, 13, "128x64 tiles"), (200, 13, "convTapWindowKernel<3x3 fp16, BN=192")]),
+    (448, [(36, 19, "BN=64, one board"), (40, 19, "128x64 tiles"), (56, 19, "BN=64, one board")]),
+    (512, [(8, 19, "64x64 tiles"), (16, 19, "half a board per workgroup, 32-row"), (60, 13, "64x64 tiles"),
+           (80, 13, "convTapWindowKernel<3x3 fp16, BN=128")]),
+    (768, [(2, 19, "32x64 tiles"), (8, 19, "half a board per workgroup, 32-row"), (22, 19, "BN=128, one board"),
+           (32, 18, "convTapWindowKernel<3x3 fp16, BN=128"), (44, 19, "BN=192, one board")]),
+    (832, [(20, 19, "half a board per workgroup, 96-row")]),
+    (1024, [(16, 13, "32x64 tiles"), (20, 13, "convTapWindowKernel<3x3 fp16, BN=128"), (3, 25, "convMfmaKernel")]),
+]
+
+
+@pytest.mark.parametrize("c,choices", CHOICES, ids=lambda v: str(v) if isinstance(v, int) else "")
+def test_built_in_choice_for_wide_convs(model_dir, c, choices):
+    """The kernel that measured fastest runs, and gives the tile kernel's bits."""
+    lm = nn.LoadedModel(modelgen.write_model(_block(c), 57, f"{model_dir}/block{c}.bin"))
+    model = nn.DeviceModel(lm, use_fp16=True)
+    for n, x, kernel in choices:
+        h = nn.DeviceHandle(model, n, x, x)
+        sp, gl = modelgen.synthetic_inputs(9, n, x, x, board_sizes=(x, x - 1))
+        dev = [nn.DeviceBuffer.from_array(r) for r in (sp, gl, np.zeros(n, np.int32), np.zeros(n, np.float32))]
+        out = nn.DeviceBuffer(n * h.row_floats * 4)
+
+        def forward():
+            h.forward_device(n, *[b.ptr for b in dev], out.ptr)
+            h.synchronize()
+            return out.to_array(np.float32, (n, h.row_floats))
+
+        h.set_profiling(True)
+        got = forward()
+        names = [r[4] for r in h.profile_kernels() if r[0] == 0]
+        h.set_profiling(False)
+        assert any(kernel in k for k in names), (n, x, kernel, names)
+        h.set_tuning("".join(f"3 3 {k} {c} {n * x * x} 0 {r} 0 {TILE_64}\n" for k in (32, c) for r in (0, 1)))
+        assert np.array_equal(forward(), got), (n, x, kernel)
         h.close()
