@@ -553,17 +553,26 @@ void launchStreamParts(const half_t* x, int cinStride, int cinPad, int cout, con
 }
 
 // 1x1: every shape below 24 row tiles of 192 (a few boards: t12d384h6 at four,
-// forwards 742 -> 652 us); beyond that plain outputs of at most 384 input
-// channels while the 32 x 64 tiles number at most 4400. b18c384nbt's 192 ->
-// 384 and 384 -> 192 convs against the 192- and 384-row DMA tiles, us per
-// forward: -39 and -48 at 24 boards, -25 and -17 at 64, -17 and +15 at 128.
-// From that row count on, gated outputs and K = 1024 are faster on the DMA
-// tiles (t12d384h6 at 16 boards). 64-row tiles for K <= 192 once the 32-row
+// forwards 742 -> 652 us). From there on the DMA kernel takes gated outputs and
+// K = 1024 (t12d384h6 at 16 boards); else the line follows K. Up to 192 input
+// channels the streamed kernel is faster at every size: a tile holds all of K
+// in little LDS, many workgroups share a CU, and the residual's load hides
+// behind the others' work (192 -> 384 with a residual against the DMA tiles,
+// us per forward of 17 of them: 80 boards -119, 128 -41, 160 -301, 256 -43; 512
+// boards 13x13 -125; 128 -> 256, 192 boards, four of them -43). Above, its
+// columns' re-reads of the rows grow with K: up to 4400 tiles (384 -> 192: 128
+// boards, 4332 tiles, -40 of 18; 160 boards, 5415, +52; 256 -> 512, 48 boards,
+// 4336, -4 of four; 64 boards, 5776, +8), and up to 2200 with a masked residual,
+// which is read in the epilogue (384 -> 384 of t12d384h6, 12 of them against the
+// 192-row DMA tiles: 24 boards, 1626 tiles, -10; 32 boards, 2166, +3; 40 boards,
+// 2712, +21; 64 boards, 4332, +30). 64-row tiles for K <= 192 once the 32-row
 // tiles number more than two per CU: half the weight reads.
 int streamTile1x1(int cinStride, int cinPad, int cout, BoardGeom g, const ConvEpilogue<half_t>& epi) {
   const long M = (long)g.batch * g.H * g.W;
   const long tiles = (M + 31) / 32 * (cout / 64);
-  if(M >= 24L * 192 && (epi.glu || cinPad > 384 || tiles > 4400)) return CONV_AUTO;
+  if(M >= 24L * 192) {
+    if(epi.glu || cinPad > 384 || tiles > (epi.maskResidualAdd ? 2200 : cinPad > 192 ? 4400 : LONG_MAX)) return CONV_AUTO;
+  }
   const int v = cinPad <= 192 && tiles > 512 ? CONV_STREAM1_64 : CONV_STREAM1_32;
   return streamFits(v, cinStride, cinPad, cout, g, epi) ? v : CONV_AUTO;
 }

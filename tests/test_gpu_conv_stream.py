@@ -5,6 +5,8 @@ outputs are the same bits. Row counts are below, at and one past 32, 64, 128
 and 192; boards are one column wide, one row high, rectangular, or wider than
 19; channel counts give one to twelve 32-channel chunks and one or several
 column tiles."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -78,27 +80,60 @@ CHOICES = [
 ]
 
 
+def _run(model, n, x, kind):
+    """A forward by the built-in choice: handle, outputs, a function that runs
+    it again, and the kernels of the kind's launches by name."""
+    h = nn.DeviceHandle(model, n, x, x)
+    sp, gl = modelgen.synthetic_inputs(9, n, x, x, board_sizes=(x, x - 1))
+    dev = [nn.DeviceBuffer.from_array(r) for r in (sp, gl, np.zeros(n, np.int32), np.zeros(n, np.float32))]
+    out = nn.DeviceBuffer(n * h.row_floats * 4)
+
+    def forward():
+        h.forward_device(n, *[b.ptr for b in dev], out.ptr)
+        h.synchronize()
+        return out.to_array(np.float32, (n, h.row_floats))
+
+    h.set_profiling(True)
+    got = forward()
+    launches = {r[4]: r[1] for r in h.profile_kernels() if r[0] == kind}
+    h.set_profiling(False)
+    return h, got, forward, launches
+
+
 @pytest.mark.parametrize("c,choices", CHOICES, ids=lambda v: str(v) if isinstance(v, int) else "")
 def test_built_in_choice_for_wide_convs(model_dir, c, choices):
     """The kernel that measured fastest runs, and gives the tile kernel's bits."""
     lm = nn.LoadedModel(modelgen.write_model(_block(c), 57, f"{model_dir}/block{c}.bin"))
     model = nn.DeviceModel(lm, use_fp16=True)
     for n, x, kernel in choices:
-        h = nn.DeviceHandle(model, n, x, x)
-        sp, gl = modelgen.synthetic_inputs(9, n, x, x, board_sizes=(x, x - 1))
-        dev = [nn.DeviceBuffer.from_array(r) for r in (sp, gl, np.zeros(n, np.int32), np.zeros(n, np.float32))]
-        out = nn.DeviceBuffer(n * h.row_floats * 4)
-
-        def forward():
-            h.forward_device(n, *[b.ptr for b in dev], out.ptr)
-            h.synchronize()
-            return out.to_array(np.float32, (n, h.row_floats))
-
-        h.set_profiling(True)
-        got = forward()
-        names = [r[4] for r in h.profile_kernels() if r[0] == 0]
-        h.set_profiling(False)
-        assert any(kernel in k for k in names), (n, x, kernel, names)
+        h, got, forward, launches = _run(model, n, x, 0)
+        assert any(kernel in k for k in launches), (n, x, kernel, launches)
         h.set_tuning("".join(f"3 3 {k} {c} {n * x * x} 0 {r} 0 {TILE_64}\n" for k in (32, c) for r in (0, 1)))
         assert np.array_equal(forward(), got), (n, x, kernel)
+        h.close()
+
+
+T384 = dataclasses.replace(modelgen.transformer_d384(), name="t2d384", blocks=["attention", "ffn"])
+
+
+@pytest.mark.parametrize("arch,cases", [
+    # (boards, side, launches of the streamed kernel, of those on 64-row tiles):
+    # post convs of 192 input channels always, pre convs of 384 up to 4400
+    # tiles, the heads' conv.
+    (_nbt(384, 192), [(16, 19, 5, 2), (128, 19, 5, 2), (160, 19, 3, 2)]),
+    # every GEMM; from 24 tiles of 192 rows no gated one nor K = 1024, [Q|K|V] up
+    # to 4400 tiles, the masked residual up to 2200; the heads' conv.
+    (T384, [(12, 19, 5, 0), (16, 19, 3, 0), (32, 19, 2, 0), (40, 19, 1, 0)]),
+], ids=["nbt", "transformer"])
+def test_built_in_choice_for_1x1_convs(model_dir, arch, cases):
+    lm = nn.LoadedModel(modelgen.write_model(arch, 57, f"{model_dir}/{arch.name}-1x1.bin"))
+    model = nn.DeviceModel(lm, use_fp16=True)
+    for n, x, streamed, rows64 in cases:
+        h, got, forward, launches = _run(model, n, x, 1)
+        count = lambda name: sum(v for k, v in launches.items() if k.startswith("convStreamKernel") and name in k)
+        assert (count(""), count("64x64")) == (streamed, rows64), (n, x, launches)
+        h.set_tuning("")
+        shapes = [l.split()[:8] for l in h.autotune(1).splitlines() if l.startswith("1 1 ")]
+        h.set_tuning("".join(" ".join(s) + f" {TILE_64}\n" for s in shapes))
+        assert np.array_equal(forward(), got), (n, x)
         h.close()
