@@ -252,6 +252,9 @@ int kgh_handle_autotune(kgh_handle* handle, int32_t reps, char* report, int32_t 
  * to its shape at launch time falls back to the built-in choice. */
 int kgh_handle_set_tuning(kgh_handle* handle, const char* table);
 int kgh_handle_get_tuning(kgh_handle* handle, char* buf, int32_t buflen);
+/* Identifies the conv kernels a table may name and the built-in choices it was
+ * measured against; a saved table of another value should be measured again. */
+uint64_t kgh_tuning_kernels(void);
 
 /* Low-latency mode for small batches (config key hipLowLatency of the
  * NeuralNet backend; no counterpart in nninterface.h): every fp16 3x3 conv

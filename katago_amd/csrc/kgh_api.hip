@@ -2166,6 +2166,8 @@ int kgh_handle_set_low_latency(kgh_handle* handle, int32_t enabled) {
   });
 }
 
+uint64_t kgh_tuning_kernels(void) { return kgh::convKernelSet(); }
+
 int kgh_handle_get_tuning(kgh_handle* handle, char* buf, int32_t buflen) {
   return guarded([&] {
     requireHandle(handle);

@@ -338,6 +338,9 @@ namespace kgh {
 // prepareConvWeights into layout [tap][cout][cinPad]; dispatches to the
 // matrix-core kernel when the shape allows, else to the direct kernel.
 const char* convVariantName(int variant);
+// A hash of the names of the kernels there are and of the built-in choice's
+// revision (see kgh_tuning_kernels).
+uint64_t convKernelSet();
 
 // variant pins the kernel when it applies to the shape; otherwise (or with
 // CONV_AUTO) the heuristic picks.

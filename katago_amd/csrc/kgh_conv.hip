@@ -1814,12 +1814,24 @@ bool convMfmaSupported(int cinPad, int cout) {
 const char* convVariantName(int variant) {
   static const char* names[] = {"auto", "tw192", "tw128", "tw64", "tw8w192", "dma1x1_192", "dma1x1_128", "dma1x1_64",
                                 "tile192", "tile128", "tile96", "tile64", "tile32", "board192", "board128", "board64",
-                                "dma1x1h_192", "dma1x1h_128", "dma1x1h_64", "boardhalf64", "allk1x1_64", "allk1x1_32",
-                                "dma1x1_256glu", "boardhalf64t32", "boardhalf192",
+                                "dma1x1h_192", "dma1x1h_128", "dma1x1h_64", "boardhalf64", "retired", "allk1x1_32",
+                                "dma1x1_256glu", "boardhalf64t32", "retired",
                                 "stream3_32", "stream3_64", "stream3_128", "stream3_192", "stream1_32", "stream1_64",
                                 "split3_32", "split3_64", "split3_96", "split1_k", "split1_wide"};
   static_assert(sizeof(names) / sizeof(names[0]) == CONV_VARIANT_COUNT, "a name per variant");
   return variant >= 0 && variant < CONV_VARIANT_COUNT ? names[variant] : "?";
+}
+
+// Raise with every change of the built-in choice or of a kernel's speed.
+constexpr int CONV_CHOICE_REVISION = 2;
+uint64_t convKernelSet() {
+  uint64_t h = 14695981039346656037ull;  // FNV-1a
+  auto add = [&](const std::string& s) {
+    for(unsigned char c : s + '\n') h = (h ^ c) * 1099511628211ull;
+  };
+  add(std::to_string(CONV_CHOICE_REVISION));
+  for(int v = 0; v < CONV_VARIANT_COUNT; v++) add(convVariantName(v));
+  return h;
 }
 
 // Conditions every matrix-core kernel needs: the epilogue moves 16 channels

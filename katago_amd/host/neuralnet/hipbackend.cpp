@@ -30,7 +30,11 @@
 #include "katago_hip_backend.h"
 
 static const int HIP_TUNER_VERSION = 1;
-static const char* HIP_TUNER_VERSION_LINE = "VERSION=2";
+
+// First line of a saved table: its format, and the kernels it was measured on.
+static std::string tunerVersionLine() {
+  return Global::strprintf("VERSION=2 KERNELS=%016llx", (unsigned long long)kgh_tuning_kernels());
+}
 
 using std::string;
 using std::vector;
@@ -403,7 +407,8 @@ void NeuralNet::freeLoadedModel(LoadedModel* loadedModel) { delete loadedModel; 
 const ModelDesc& NeuralNet::getModelDesc(const LoadedModel* loadedModel) { return loadedModel->modelDesc; }
 
 // Tile choices for the handle's batch size: read from the tuning file when
-// one exists, else measured on the device (kgh_handle_autotune) and saved.
+// one exists, else measured on the device (kgh_handle_autotune) and saved. A
+// file of another kernel set is measured again and replaced.
 // Batches of 8 boards or fewer keep the built-in choices.
 static void maybeAutoTune(ComputeHandle& h, Logger* logger, int serverThreadIdx) {
   ComputeContext& c = *h.context;
@@ -427,8 +432,8 @@ static void maybeAutoTune(ComputeHandle& h, Logger* logger, int serverThreadIdx)
       std::stringstream ss;
       ss << in.rdbuf();
       string text = ss.str();
-      if(text.rfind(HIP_TUNER_VERSION_LINE, 0) == 0) {
-        const size_t eol = text.find('\n');
+      const size_t eol = text.find('\n');
+      if(text.substr(0, eol) == tunerVersionLine()) {
         const string table = eol == string::npos ? string() : text.substr(eol + 1);
         checkKgh(kgh_handle_set_tuning(h.handle, table.c_str()), "kgh_handle_set_tuning");
         h.tuningSource = 1;
@@ -440,7 +445,7 @@ static void maybeAutoTune(ComputeHandle& h, Logger* logger, int serverThreadIdx)
   vector<char> report(1 << 16);
   checkKgh(kgh_handle_autotune(h.handle, 3, report.data(), (int32_t)report.size()), "kgh_handle_autotune");
   h.tuningSource = 2;
-  string text = string(HIP_TUNER_VERSION_LINE) + "\n# ky kx cinPad cout M gated residual maskedResidual variant name best_us heuristic_us\n" +
+  string text = tunerVersionLine() + "\n# ky kx cinPad cout M gated residual maskedResidual variant name best_us heuristic_us\n" +
                 report.data();
   // Save atomically; a directory that cannot be written only costs re-tuning.
   mkdir(c.tunerDir.c_str(), 0755);

@@ -79,6 +79,27 @@ def test_explicit_tuner_file_and_small_batches(model_dir, tmp_path):
         assert np.array_equal(x[k], y[k]), k
 
 
+def test_table_of_other_kernels_is_measured_again(model_dir, tmp_path):
+    """A saved table is loaded only if its first line names the kernels there
+    are now: one from before a change of them would go on pinning its shapes to
+    kernels that are no longer the fastest."""
+    lm = nn.LoadedModel(modelgen.ensure_model(model_dir, modelgen.configs()[0]))
+    path = str(tmp_path / "tuning.txt")
+
+    def source():
+        h = nn.ComputeHandle(nn.ComputeContext(lm, use_fp16=False, auto_tune=True, tuner_file=path), max_batch=16)
+        return h.tuning()[0]
+
+    assert source() == 2 and source() == 1
+    text = open(path).read()
+    first, table = text.split("\n", 1)
+    for other in ("VERSION=2", first[:-1] + ("0" if first[-1] != "0" else "1"), first + "0", "VERSION=1"):
+        open(path, "w").write(other + "\n" + table)
+        assert source() == 2, other
+        assert open(path).read().split("\n", 1)[0] == first
+    assert source() == 1
+
+
 @pytest.mark.parametrize("fp16", [True, False], ids=["fp16", "fp32"])
 def test_every_kernel_variant_gives_identical_bits(model_dir, fp16):
     """Pin every shape to each variant in turn (a variant that does not apply
