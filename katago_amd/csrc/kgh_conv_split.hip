@@ -20,8 +20,14 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // share a second set, so a sum is rounded at its own magnitude once per 16
 // channels.
 //
-// An infinite input gives NaN (its rest is), where products in fp32 gave an
-// infinity or NaN.
+// A finite number that rounds to a bf16 infinity has the largest bf16 number as
+// its first piece, and an infinity has only a third, so that it meets one piece
+// of the other factor, the one with that factor's sign: sums are infinite or NaN
+// as they are in fp32 (but NaN where both factors are infinite, and a finite sum
+// within 2^-8 of the largest float may already be infinite). A wave that sees
+// such a number splits its part of the panel a second time; looking for them
+// costs 2 us of b6c96's 187 at eight boards, 10 of b18c384nbt's 1323 at one and
+// 8 of its 2760 at 16 (in the first pass, without a second, 20 to 25 of each).
 //
 // K (16-channel chunk outer, tap inner) is cut into four groups of whole
 // chunks, summed ((p0 + p1) + p2) + p3, by four waves at once or by one wave
@@ -60,20 +66,40 @@ struct SplitDims {
   int colTiles;
 };
 
-// The three pieces of eight floats, to dst, dst + 32 and dst + 64.
-__device__ __forceinline__ void storePieces(unsigned char* dst, const float4 (&v)[2]) {
+constexpr float BF16_MAX = 0x1.fep127f, BF16_INF_FROM = 0x1.ffp127f;  // rounds to infinity from there
+
+// Piece q of what the pieces before it left of a float; SPECIAL also splits
+// infinities and what rounds to one.
+template<bool SPECIAL>
+__device__ __forceinline__ __bf16 nextPiece(int q, float rest) {
+  if(SPECIAL && q < 2 && fabsf(rest) >= BF16_INF_FROM) return (__bf16)(fabsf(rest) == INFINITY ? 0.0f : copysignf(BF16_MAX, rest));
+  return (__bf16)rest;
+}
+
+// The three pieces of eight floats, to dst, dst + 32 and dst + 64; or-s the
+// last one's bits into seen.
+template<bool SPECIAL>
+__device__ __forceinline__ void storePieces(unsigned char* dst, const float4 (&v)[2], unsigned& seen) {
   float rest[8] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w};
+  union {
+    bf16x8 p;
+    uint4 bits;
+  } piece;
 #pragma unroll
   for(int q = 0; q < 3; q++) {
-    bf16x8 p;
 #pragma unroll
     for(int j = 0; j < 8; j++) {
-      p[j] = (__bf16)rest[j];
-      rest[j] -= (float)p[j];
+      piece.p[j] = nextPiece<SPECIAL>(q, rest[j]);
+      rest[j] -= (float)piece.p[j];
     }
-    *(bf16x8*)(dst + q * 32) = p;
+    *(uint4*)(dst + q * 32) = piece.bits;
   }
+  seen |= piece.bits.x | piece.bits.y | piece.bits.z | piece.bits.w;
 }
+// What is or rounds to an infinity leaves a NaN in the last piece, whose
+// exponent has its highest bit set; so have third pieces of 2 and more, of
+// numbers from 2^18, which are split the same way again.
+__device__ __forceinline__ bool anySpecial(unsigned seen) { return __any(seen & 0x40004000u); }
 
 // One K step of RB row blocks: six products each. A piece's registers take
 // the next step's right after its last use here (a step starts with the piece
@@ -187,8 +213,10 @@ __global__ __launch_bounds__(64 * WN * SPLIT_GROUPS, 1) void convSplitKernel(con
   // feed taps that read zeros, or outputs that are never stored: they load a
   // valid address, as do the slots past the last row or the group's last
   // chunk, which are not written.
-  auto loadPanel = [&](int first) {
-    constexpr int U = 4;
+  auto loadPanel = [&](int first, auto specialTag) {
+    constexpr bool SPECIAL = decltype(specialTag)::value;
+    constexpr int U = SPECIAL ? 1 : 4;
+    unsigned seen = 0;
     const int groupSlots = sd.panel * 2;
     const int per = KW * groupSlots;
     const int total = winRows * per;
@@ -211,8 +239,9 @@ __global__ __launch_bounds__(64 * WN * SPLIT_GROUPS, 1) void convSplitKernel(con
       }
 #pragma unroll
       for(int u = 0; u < U; u++)
-        if(dst[u] >= 0) storePieces(win + dst[u], val[u]);
+        if(dst[u] >= 0) storePieces<SPECIAL>(win + dst[u], val[u], seen);
     }
+    return seen;
   };
 
   floatx16 lead[RB], small[RB], sum[RB];
@@ -231,7 +260,7 @@ __global__ __launch_bounds__(64 * WN * SPLIT_GROUPS, 1) void convSplitKernel(con
 #pragma unroll
       for(int q = 0; q < 3; q++) bRing[d][q] = readB(s0 + min(d, sLast), q);
     if(first > 0) __syncthreads();  // every wave is done with the panel before
-    loadPanel(first);
+    if(__builtin_expect(anySpecial(loadPanel(first, std::false_type())), 0)) loadPanel(first, std::true_type());
     __syncthreads();
     if(pc == 0) continue;
 #pragma unroll
@@ -348,8 +377,10 @@ __global__ __launch_bounds__(512, 2) void convSplitWideKernel(const float* __res
 #pragma unroll
       for(int q = 0; q < 3; q++) bRing[d][q] = readB(c0 + min(d, pc - 1), q);
     if(c0 > 0) __syncthreads();  // every wave is done with the panel before
-    {
-      constexpr int U = 4;
+    auto loadPanel = [&](auto specialTag) {
+      constexpr bool SPECIAL = decltype(specialTag)::value;
+      constexpr int U = SPECIAL ? 1 : 4;
+      unsigned seen = 0;
       const int per = sd.panel * 2;
       const int total = BM * per;
       for(int base = 0; base < total; base += U * NT) {
@@ -369,9 +400,11 @@ __global__ __launch_bounds__(512, 2) void convSplitWideKernel(const float* __res
         }
 #pragma unroll
         for(int u = 0; u < U; u++)
-          if(dst[u] >= 0) storePieces(win + dst[u], val[u]);
+          if(dst[u] >= 0) storePieces<SPECIAL>(win + dst[u], val[u], seen);
       }
-    }
+      return seen;
+    };
+    if(__builtin_expect(anySpecial(loadPanel(std::false_type())), 0)) loadPanel(std::true_type());
     __syncthreads();
     if(!live) continue;
 #pragma unroll
@@ -417,7 +450,7 @@ __global__ void prepareSplitWeightsKernel(const float* __restrict__ src, __bf16*
   const int ic = (int)(step / taps) * 16 + (lane >> 5) * 8 + (int)(idx & 7);
   float rest = ic < cin ? src[(((size_t)oc * cin + ic) * ks + tap / ks) * ks + tap % ks] : 0.0f;
   for(int q = 0; q < 3; q++) {
-    const __bf16 p = (__bf16)rest;
+    const __bf16 p = nextPiece<true>(q, rest);
     dst[blk * 1536 + q * 512 + (idx & 511)] = p;
     rest -= (float)p;
   }

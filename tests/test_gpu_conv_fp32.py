@@ -40,3 +40,46 @@ def test_rows_do_not_depend_on_batch(model_dir, arch):
         got = h.get_output(sp[:n], gl[:n])
         for k in want:
             assert np.array_equal(got[k], want[k][:n]), (n, k)
+
+
+def _conv_text(w):
+    return "c %d %d %d %d 1 1\n%s\n" % (*w.shape, " ".join(repr(float(v)) for v in w.reshape(-1)))
+
+
+def _conv(x, w):
+    """The device's conv of x [n, y, x, cin] with w [ky, kx, cin, cout]."""
+    n, h, wd, _ = x.shape
+    out = nn.test_evaluate(nn.TEST_CONV, _conv_text(w), n, wd, h, False, True, x, None, w.shape[3])
+    return out.reshape(n, h, wd, w.shape[3])
+
+
+def _conv64(x, w, dtype=np.float64):
+    """The same as a sum of products in float64 (or float32, in some order)."""
+    k = w.shape[0]
+    xp = np.pad(x.astype(dtype), ((0, 0), (k // 2, k // 2), (k // 2, k // 2), (0, 0)))
+    h, wd = x.shape[1:3]
+    with np.errstate(all="ignore"):
+        return sum(xp[:, dy:dy + h, dx:dx + wd] @ w[dy, dx].astype(dtype) for dy in range(k) for dx in range(k))
+
+
+SHAPES = [(3, 32, 32, 1, 9), (3, 64, 64, 2, 19), (3, 192, 64, 16, 19), (3, 96, 64, 40, 19), (1, 384, 192, 1, 19), (1, 192, 384, 30, 19)]
+
+
+@pytest.mark.parametrize("k,cin,cout,n,side", SHAPES, ids=str)
+def test_infinite_and_largest_inputs(k, cin, cout, n, side):
+    """Infinities, NaN and numbers past the largest bf16 (and past the last that
+    rounds to it) among ordinary ones: sums are infinite and NaN where a float32
+    conv's are, the others are right to 1e-5 of the sum of their terms' sizes."""
+    rng = np.random.default_rng(k + cin)
+    x = rng.standard_normal((n, side, side, cin)).astype(np.float32)
+    w = (rng.standard_normal((k, k, cin, cout)) / cin).astype(np.float32)
+    for i, v in enumerate((np.inf, -np.inf, np.nan, 3.4028235e38, -3.4e38, 3.396e38, 3.39e38)):
+        x[0, (i * 2) % side, (i * 3) % side, (i * 5) % cin] = v
+    got, want = _conv(x, w), _conv64(x, w)
+    assert np.isinf(want).any() and np.isnan(want).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf].astype(np.float32))
+    fin = np.isfinite(want)
+    size = _conv64(np.abs(np.where(np.isfinite(x), x, 0)), np.abs(w))
+    assert np.isfinite(got[fin]).all() and (np.abs(got[fin] - want[fin]) <= 1e-5 * size[fin]).all()
