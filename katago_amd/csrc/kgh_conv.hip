@@ -1859,7 +1859,7 @@ bool convVariantApplies(int variant, const T* x, int cinStride, int cinPad, int 
            variantFits(variant, ky, cinStride, cinPad, cout, g, epi);
   else
     return mfmaPathOk<T>(cinStride, cinPad, cout, ky, kx, wPrepared, epi) && kgh::splitFits(ky, cinStride, cinPad, cout, epi) &&
-           kgh::splitVariantFits(variant, ky, cout);
+           kgh::splitVariantFits(variant, ky, cout, g);
 }
 
 template<typename T>
@@ -1887,8 +1887,11 @@ void launchConv(const T* x, int cinStride, int cin, int cinPad, int cout, int ky
     throw KghError(5, "conv: a rotary embedding in the epilogue needs the matrix-core kernels and head dims multiples of 16");
   bool done = false;
   if constexpr(std::is_same<T, float>::value) {
-    if(mfmaPathOk<T>(cinStride, cinPad, cout, ky, kx, wPrepared, epi) && kgh::splitFits(ky, cinStride, cinPad, cout, epi)) {
-      if(!kgh::splitVariantFits(variant, ky, cout)) variant = kgh::splitChoice(ky, cout, g);
+    // Boards too wide for its window (only layers by themselves have them) take
+    // the direct kernel.
+    if(mfmaPathOk<T>(cinStride, cinPad, cout, ky, kx, wPrepared, epi) && kgh::splitFits(ky, cinStride, cinPad, cout, epi) &&
+       kgh::splitBoardFits(ky, g)) {
+      if(!kgh::splitVariantFits(variant, ky, cout, g)) variant = kgh::splitChoice(ky, cout, g);
       kgh::launchSplit(variant, x, cinStride, cinPad, cout, (const float*)wPrepared, g, epi, stream);
       done = true;
     }
@@ -1911,6 +1914,7 @@ void launchConv(const T* x, int cinStride, int cin, int cinPad, int cout, int ky
   }
   if(usedMfma != nullptr) *usedMfma = done;
   if(done) return;
+  if(epi.sumSqOut != nullptr) throw KghError(5, "conv: board too wide for the fp32 kernel that records sums of squares");
   if(wDirect == nullptr) throw KghError(5, "conv: no direct-layout weights for a shape the matrix-core kernel does not take");
   int threads = 256;
   if(epi.glu) {

@@ -8,11 +8,13 @@ namespace kgh {
 
 extern thread_local const char* g_lastConvKernel;
 
-// Whether they take a ks x ks conv, whatever its batch.
+// Whether they take a ks x ks conv, whatever its batch, and one on boards of
+// this size.
 bool splitFits(int ks, int cinStride, int cinPad, int cout, const ConvEpilogue<float>& epi);
+bool splitBoardFits(int ks, BoardGeom g);
 // Whether a tile (ConvVariant CONV_SPLIT*) takes such a conv, and the one the
 // built-in choice runs. All of them give the same bits.
-bool splitVariantFits(int variant, int ks, int cout);
+bool splitVariantFits(int variant, int ks, int cout, BoardGeom g);
 int splitChoice(int ks, int cout, BoardGeom g);
 // Runs one; w are the split weights.
 void launchSplit(int variant, const float* x, int cinStride, int cinPad, int cout, const float* w, BoardGeom g,

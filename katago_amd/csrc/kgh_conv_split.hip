@@ -456,6 +456,10 @@ __global__ void prepareSplitWeightsKernel(const float* __restrict__ src, __bf16*
   }
 }
 
+// Rows of a window (and the row of zeros), and the bytes of one.
+long splitWindowRows(int ks, int rows, int W) { return rows + (ks == 3 ? 2 * (W + 1) + 1 : 0); }
+int splitRowBytes(int panel) { return SPLIT_GROUPS * panel * 96 + 16; }
+
 template<int KS, int RB, int WN>
 void launchTile(const float* x, int cinStride, int cinPad, int cout, const __bf16* wf, BoardGeom g, const ConvEpilogue<float>& epi,
                 hipStream_t stream) {
@@ -465,8 +469,7 @@ void launchTile(const float* x, int cinStride, int cinPad, int cout, const __bf1
   const int M = g.batch * g.H * g.W;
   const int colTiles = cout / (32 * WN);
   const long tiles = (long)((M + BM - 1) / BM) * colTiles;
-  const int winRows = BM + (KS == 3 ? 2 * (g.W + 1) : 0);
-  const int rows = winRows + (KS == 3 ? 1 : 0);
+  const int rows = (int)splitWindowRows(KS, BM, g.W);
   const int fixed = KS == 1 ? BM * 4 : 0;
   const int sums = KW * RB * WN * SPLIT_PART_BYTES + RB * WN * SPLIT_STAGE_BYTES;
   // The largest panel in the LDS of a CU, or in half of it where there are two
@@ -477,7 +480,7 @@ void launchTile(const float* x, int cinStride, int cinPad, int cout, const __bf1
   const int most = std::max((budget / rows - 16) / (96 * KW), 1);
   const int panels = (group + most - 1) / most;
   const int panel = (group + panels - 1) / panels;
-  const int lds = fixed + std::max(rows * (96 * KW * panel + 16), sums);
+  const int lds = fixed + std::max(rows * splitRowBytes(panel), sums);
   if(lds > SPLIT_MAX_LDS) throw KghError(5, "conv: board too wide for the fp32 kernel");
   const SplitDims sd = {panel, panels, splitMagic(KW * panel * 2), splitMagic(panel * 2), splitMagic(g.H * g.W), splitMagic(g.W), colTiles};
   const dim3 grid((unsigned)tiles), block(64 * WN * KW);
@@ -520,8 +523,20 @@ bool splitFits(int ks, int cinStride, int cinPad, int cout, const ConvEpilogue<f
          (ks == 1 || (!epi.glu && epi.rowNormIn == nullptr && epi.ropeEnd == 0));
 }
 
-bool splitVariantFits(int variant, int ks, int cout) {
-  if(ks == 3) return variant == CONV_SPLIT3_32 || (cout % 64 == 0 && (variant == CONV_SPLIT3_64 || variant == CONV_SPLIT3_96));
+// 3x3: a tile's window with one chunk of each K group in the LDS (boards up to
+// 187 wide on 32-row tiles, 155 on 96), and positions of a board within the
+// exact range of the divisions by multiplication.
+static bool windowFits(int rows, BoardGeom g) {
+  const long hw = (long)g.H * g.W;
+  return splitWindowRows(3, rows, g.W) * splitRowBytes(1) <= SPLIT_MAX_LDS && 4 * (hw + 96) * hw < (1L << 32);
+}
+bool splitBoardFits(int ks, BoardGeom g) { return ks == 1 || windowFits(32, g); }
+
+bool splitVariantFits(int variant, int ks, int cout, BoardGeom g) {
+  if(ks == 3) {
+    if(variant == CONV_SPLIT3_32) return windowFits(32, g);
+    return cout % 64 == 0 && ((variant == CONV_SPLIT3_64 && windowFits(64, g)) || (variant == CONV_SPLIT3_96 && windowFits(96, g)));
+  }
   return variant == CONV_SPLIT1_K || variant == CONV_SPLIT1_WIDE;
 }
 
@@ -540,7 +555,7 @@ int splitChoice(int ks, int cout, BoardGeom g) {
   const int cols = cout % 64 == 0 ? 64 : 32;
   auto tiles = [&](int rows) { return (M + rows - 1) / rows * (cout / cols); };
   if(ks == 1) return tiles(32) > 512 ? CONV_SPLIT1_WIDE : CONV_SPLIT1_K;
-  if(cols == 32 || tiles(32) <= 256) return CONV_SPLIT3_32;
+  if(cols == 32 || tiles(32) <= 256 || !windowFits(96, g)) return CONV_SPLIT3_32;
   return tiles(64) <= 256 ? CONV_SPLIT3_64 : CONV_SPLIT3_96;
 }
 

@@ -83,3 +83,15 @@ def test_infinite_and_largest_inputs(k, cin, cout, n, side):
     fin = np.isfinite(want)
     size = _conv64(np.abs(np.where(np.isfinite(x), x, 0)), np.abs(w))
     assert np.isfinite(got[fin]).all() and (np.abs(got[fin] - want[fin]) <= 1e-5 * size[fin]).all()
+
+
+@pytest.mark.parametrize("x,y,n", [(155, 2, 1), (156, 2, 60), (187, 3, 1), (188, 3, 1), (300, 2, 2), (182, 181, 1)], ids=str)
+def test_boards_wider_than_a_window(x, y, n):
+    """A conv by itself on boards at and past the widest that the tiles' windows
+    hold (155 for 96 rows, 187 for 32), and of more positions than their
+    divisions take: the direct kernel has those."""
+    rng = np.random.default_rng(x)
+    inp = rng.standard_normal((n, y, x, 32)).astype(np.float32)
+    w = (rng.standard_normal((3, 3, 32, 64)) / 17).astype(np.float32)
+    got, want = _conv(inp, w), _conv64(inp, w)
+    assert np.abs(got - want).max() <= 1e-5
