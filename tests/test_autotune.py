@@ -121,29 +121,50 @@ def test_every_kernel_variant_gives_identical_bits(model_dir, fp16):
             assert np.array_equal(out[k], ref[k]), (v, k)
 
 
-@pytest.mark.parametrize("variant", [16, 17, 18, 20, 21, 13, 15, 19, 23, 24],
-                         ids=["dma1x1h_192", "dma1x1h_128", "dma1x1h_64", "allk1x1_64", "allk1x1_32", "board192", "board64",
-                              "boardhalf64", "boardhalf64t32", "boardhalf192"])
-def test_variants_give_identical_bits_on_nbt(model_dir, variant):
+NBT_VARIANTS = {13: "convBoardWindowKernel<3x3 fp16, BN=192, one", 15: "convBoardWindowKernel<3x3 fp16, BN=64, one",
+                16: "conv1x1DmaKernel<1x1 fp16, BN=192, BM=192", 17: "conv1x1DmaKernel<1x1 fp16, BN=128, BM=192",
+                18: "conv1x1DmaKernel<1x1 fp16, BN=64, BM=192", 19: "half a board per workgroup, 96-row wave",
+                21: "conv1x1AllKKernel", 23: "half a board per workgroup, 32-row wave", 25: "<3x3 fp16, 32x64 tiles",
+                26: "<3x3 fp16, 64x64 tiles", 27: "<3x3 fp16, 128x64 tiles", 28: "<3x3 fp16, 192x64 tiles",
+                29: "<1x1 fp16, 32x64 tiles", 30: "<1x1 fp16, 64x64 tiles"}
+
+
+def test_variants_give_identical_bits_on_nbt(model_dir):
     """On C2's nested-bottleneck shapes (192-channel 3x3 convs, which the
     b10c128 test above cannot pin to the 192-column board kernels): the
-    192-row and whole-K 1x1 kernels, including the post 1x1 conv whose
+    192-row, whole-K and streamed 1x1 kernels, including the post 1x1 conv whose
     residual is loaded into the accumulators (through the stage that shares
-    the A buffers in the 192-row kernel), and the one-board 3x3 kernels on
-    whole and half boards: bitwise the built-in outputs."""
+    the A buffers in the 192-row kernel), the one-board 3x3 kernels on
+    whole and half boards, and the streamed ones. Each one pinned runs and gives
+    the built-in outputs' bits; an id whose kernel is gone runs the built-in
+    choice."""
     cfg = modelgen.configs()[2]
     lm = nn.LoadedModel(modelgen.ensure_model(model_dir, cfg))
-    n = 12  # batches of 8 boards or fewer are not tuned
+    n = 12
     sp, gl = modelgen.synthetic_inputs(cfg.input_seed, n, board_sizes=(19, 13))
-    tuned = nn.ComputeHandle(nn.ComputeContext(lm, use_fp16=True, auto_tune=True, tuner_file=str(model_dir) + "/t_nbt.txt"),
-                             max_batch=n)
-    shapes = [l.split()[:8] for l in tuned.tuning()[1].splitlines() if l.strip()]
+    h = nn.DeviceHandle(nn.DeviceModel(lm, use_fp16=True), n)
+    shapes = [l.split()[:8] for l in h.autotune(1).splitlines() if l.strip()]
     assert any(k[0] == "1" and k[6] == "1" for k in shapes)  # a 1x1 shape with a residual
-    ref = _forward(nn.ComputeHandle(nn.ComputeContext(lm, use_fp16=True, auto_tune=False), max_batch=n), sp, gl)
-    tuned.set_tuning("".join(" ".join(k) + f" {variant}\n" for k in shapes))
-    out = _forward(tuned, sp, gl)
-    for k in out:
-        assert np.array_equal(out[k], ref[k]), k
+    dev = [nn.DeviceBuffer.from_array(r) for r in (sp, gl, (np.arange(n) % 8).astype(np.int32), np.zeros(n, np.float32))]
+    out = nn.DeviceBuffer(n * h.row_floats * 4)
+
+    def forward(variant):
+        h.set_tuning("".join(" ".join(k) + f" {variant}\n" for k in shapes))
+        h.set_profiling(True)
+        h.forward_device(n, *[b.ptr for b in dev], out.ptr)
+        h.synchronize()
+        names = {r[4] for r in h.profile_kernels()}
+        h.set_profiling(False)
+        return out.to_array(np.float32, (n, h.row_floats)), names
+
+    ref, built_in = forward(0)
+    for variant, name in NBT_VARIANTS.items():
+        got, names = forward(variant)
+        assert any(name in k for k in names), (variant, names)
+        assert np.array_equal(got, ref), variant
+    for retired in (20, 24):
+        got, names = forward(retired)
+        assert names == built_in and np.array_equal(got, ref), retired
 
 
 def test_every_kernel_variant_gives_identical_bits_on_transformer(model_dir):

@@ -25,7 +25,7 @@ def _file(model_dir, arch):
 @pytest.mark.parametrize("arch", NETS, ids=lambda a: a.name)
 def test_edges_match_oracle(model_dir, arch, nn_x, nn_y):
     """Tolerances are _compare's fp32 bounds (1e-3 absolute on the raw
-    outputs; products are exact to 2^-24 of their terms, as in fp32)."""
+    outputs): edges and layouts; test_sums_match_float64 holds the products."""
     _run_parity(_file(model_dir, arch), False, 1, board_sizes=((nn_x, nn_y),), label=f"fp32 {nn_x}x{nn_y}", nn_x=nn_x, nn_y=nn_y)
 
 
@@ -63,6 +63,36 @@ def _conv64(x, w, dtype=np.float64):
 
 
 SHAPES = [(3, 32, 32, 1, 9), (3, 64, 64, 2, 19), (3, 192, 64, 16, 19), (3, 96, 64, 40, 19), (1, 384, 192, 1, 19), (1, 192, 384, 30, 19)]
+
+
+def _pieces(a):
+    """A float32 array as three bf16 arrays, each the rounded rest (nearest even)."""
+    out, rest = [], a.astype(np.float32)
+    for _ in range(3):
+        bits = rest.view(np.uint32).astype(np.uint64)
+        p = ((bits + 0x7FFF + ((bits >> 16) & 1)) & 0xFFFF0000).astype(np.uint32).view(np.float32)
+        out.append(p)
+        rest = rest - p
+    return out
+
+
+@pytest.mark.parametrize("k,cin,cout,n,side", SHAPES + [(3, 384, 64, 1, 19), (3, 80, 96, 3, 13), (1, 1024, 384, 4, 19), (1, 48, 96, 2, 7)], ids=str)
+def test_sums_match_float64(k, cin, cout, n, side):
+    """One conv on every tile against float64, in the 2-norm. A sum rounds once
+    per 16 channels and tap (up to 216 times), each time by 2^-24 / sqrt(12) of
+    a partial sum: 1.8e-7 if they were all of the final size; measured 0.5e-7 to
+    1.7e-7 (numpy's float32 sums 1.2e-7 to 3.6e-7). Any of the three products of
+    2^-18 left out of the six would give 1e-6 and more."""
+    rng = np.random.default_rng(k + cin)
+    x = rng.standard_normal((n, side, side, cin)).astype(np.float32)
+    w = (rng.standard_normal((k, k, cin, cout)) * np.sqrt(2.0 / (k * k * cin))).astype(np.float32)
+    want = _conv64(x, w)
+    size = np.linalg.norm(want)
+    assert np.linalg.norm(_conv(x, w) - want) <= 5e-7 * size
+    if n == 1:  # what a product left out is, on the CPU
+        a, b = _pieces(x), _pieces(w)
+        for i, j in ((0, 2), (1, 1), (2, 0)):
+            assert np.linalg.norm(_conv64(a[i], b[j])) > 1e-6 * size
 
 
 @pytest.mark.parametrize("k,cin,cout,n,side", SHAPES, ids=str)

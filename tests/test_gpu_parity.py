@@ -249,8 +249,8 @@ def _tiny_transformer(heads, kv, dq, dv, c, learnable, tip):
     (2, 1, 64, 64, 128, True, False),
 ], ids=["mha-q32v32-fixed", "gqa-q32v16-learnable", "mqa-q64v64-bntip"])
 def test_tiny_transformers_match_oracle(model_dir, heads, kv, dq, dv, c, learnable, tip, fp16):
-    """Head shapes that select each matrix-core attention variant in fp16 (and
-    the plain kernel in fp32)."""
+    """Head shapes that select each matrix-core attention variant, in fp16 and
+    in fp32."""
     arch = _tiny_transformer(heads, kv, dq, dv, c, learnable, tip)
     path = modelgen.write_model(arch, 31 + heads + dq, f"{model_dir}/{arch.name}-{learnable}-{tip}.bin.gz")
     _run_parity(path, fp16, 5, board_sizes=(19, 9, 13, 7), label=arch.name)
@@ -528,10 +528,10 @@ def test_profile_records_name_the_kernels_that_ran(model_dir):
 
 @pytest.mark.parametrize("cfg_index", [0, 1], ids=["b6c96", "b10c128"])
 def test_fp32_rows_do_not_depend_on_batch_size(model_dir, cfg_index):
-    """fp32 contexts: every 3x3 conv runs the fp32 split kernel (32 x 32
-    output blocks, K dealt over eight waves, partial sums added in wave order)
-    at every batch size, so a board's row is bitwise the same in every batch
-    that holds it, also across the 32-row block boundaries a batch moves."""
+    """fp32 contexts: every conv adds its products on the bf16 matrix cores in
+    four groups of K, summed in a fixed order whichever tile the batch size
+    selects, so a board's row is bitwise the same in every batch that holds it,
+    also across the tile boundaries a batch moves."""
     cfg = modelgen.configs()[cfg_index]
     lm = nn.LoadedModel(modelgen.ensure_model(model_dir, cfg))
     n_max = 64

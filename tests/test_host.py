@@ -171,7 +171,7 @@ def test_hot_kernels_keep_everything_in_registers():
         usage = json.load(f)
     hot = ("convBoardWindowKernel", "convTapWindowKernel", "conv1x1DmaKernel", "conv1x1AllKKernel", "convMfmaKernel", "flashAttentionKernel",
            "poolVecKernel", "headVectorKernel", "bnActVecKernel", "rmsNormRowKernel", "headSpatialKernel", "gpoolBiasActKernel",
-           "splitKEpilogueKernel")
+           "splitKEpilogueKernel", "convStreamKernel", "convSplitKernel", "convSplitWideKernel", "attentionF32Kernel")
     seen = set()
     for name, u in usage.items():
         for h in hot:
