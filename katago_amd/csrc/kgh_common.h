@@ -334,14 +334,14 @@ enum ConvVariant {
 // Host-side launchers (definitions in kgh_conv.hip / kgh_kernels.hip).
 namespace kgh {
 
-// Conv of x[M, cinStride] (first cin channels used) with weights prepared by
-// prepareConvWeights into layout [tap][cout][cinPad]; dispatches to the
-// matrix-core kernel when the shape allows, else to the direct kernel.
 const char* convVariantName(int variant);
 // A hash of the names of the kernels there are and of the built-in choice's
 // revision (see kgh_tuning_kernels).
 uint64_t convKernelSet();
 
+// Conv of x[M, cinStride] (first cin channels used) with weights prepared by
+// prepareConvWeights; dispatches to a matrix-core kernel when the shape allows,
+// else to the direct kernel with wDirect, (oc, ic, y, x) in fp32.
 // variant pins the kernel when it applies to the shape; otherwise (or with
 // CONV_AUTO) the heuristic picks.
 template<typename T>
@@ -357,12 +357,12 @@ bool convVariantApplies(int variant, const T* x, int cinStride, int cinPad, int 
 template<typename T>
 bool convMfmaSupported(int cinPad, int cout);
 
-// Whether launchConv takes the epilogue's folded-RMSNorm fields for this
-// shape (a matrix-core kernel; raw split on 32 columns; no residual where the
-// accumulators are scaled).
 // Whether epi's rotary embedding (see ConvEpilogue) can run in this conv.
 template<typename T>
 bool convRopeOk(int cinStride, int cinPad, int cout, int ky, int kx, const void* wPrepared, const ConvEpilogue<T>& epi);
+// Whether launchConv takes the epilogue's folded-RMSNorm fields for this
+// shape (a matrix-core kernel; raw split on 32 columns; no residual where the
+// accumulators are scaled).
 template<typename T>
 bool convNormFoldOk(int cinStride, int cinPad, int cout, int ky, int kx, const void* wPrepared, const ConvEpilogue<T>& epi);
 
@@ -379,14 +379,14 @@ bool convSplitKNeedsWork(int cinPad, BoardGeom g);
 void launchConvSplitK(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
                       const ConvEpilogue<half_t>& epi, float* work, hipStream_t stream);
 
-// Converts fp32 weights (oc, ic, y, x) to the kernel layout [tap][oc][cinPad]
-// of type T on device (zero-padded channels).
+// Prepares fp32 weights (oc, ic, y, x) on the device, channels zero-padded. In
+// fp16: [tap][oc][cinPad], and for 1x1 and 3x3 kernels after it the streamed
+// kernel's fragments (kgh_conv_stream.hip). In fp32: the fragments of three bf16
+// pieces (kgh_conv_split.hip).
 template<typename T>
 void prepareConvWeights(const float* dWeightsOIYX, T* dOut, int cout, int cin, int cinPad, int ky, int kx, hipStream_t stream);
-// Elements prepareConvWeights writes: ky*kx*cout*cinPad, and for fp32 3x3
-// convs with cinPad a multiple of 16 and cout of 32 as many again, the
-// layout of the fp32 3x3 kernel (each wave's weight fragments of a step one
-// contiguous 2 KB run) following the first.
+// Elements of T that prepareConvWeights writes: ky*kx*cout*cinPad, twice that
+// with fragments in fp16, 3/2 of it in fp32.
 size_t preparedConvWeightElems(bool fp16, int ky, int kx, int cout, int cinPad);
 
 template<typename T>

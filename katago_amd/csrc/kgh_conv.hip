@@ -35,7 +35,9 @@ const char* lastConvKernel() { return g_lastConvKernel; }
 
 namespace {
 
-// ROPE: the rotary-embedding mode of ConvEpilogue (raw outputs only, no
+// Epilogue of the 128-row tile kernel; requires convStageBytes(WM) bytes of LDS
+// at smem and must be reached by every thread of the workgroup (it contains
+// barriers). ROPE: the rotary-embedding mode of ConvEpilogue (raw outputs only, no
 // activated output), instantiated only in kernels that take 1x1 convs.
 template<typename T, int BN, int WM, int ACT, bool ROPE = false>
 __device__ __forceinline__ void storeTileEpilogueAct(floatx16 (&acc)[CONV_BM / WM / 32][BN / (4 / WM) / 32], unsigned char* smem,
@@ -163,14 +165,15 @@ __device__ __forceinline__ void storeTileEpilogue(floatx16 (&acc)[CONV_BM / WM /
   });
 }
 
-// Operand layout of a 32x32 matrix-core tile (both instructions above): lane l
+// Operand layout of a 32x32 matrix-core tile: lane l
 // supplies row (l % 32) of A and column (l % 32) of B for k-group (l / 32);
 // result register r of lane l holds C[(r/4)*8 + (l/32)*4 + r%4][l % 32].
-template<typename T, int KS, int BN, int WM>
+template<int KS, int BN, int WM>
 // Three workgroups per CU (<= 168 registers per lane, ~51 KB LDS each) so a
 // batch-256 19x19 launch (722 row tiles) fits the 768 slots of 256 CUs at once.
-__global__ __launch_bounds__(CONV_THREADS, 3) void convMfmaKernel(const T* __restrict__ x, int cinStride, int cinPad, int cout,
-                                                               const T* __restrict__ w, BoardGeom g, ConvEpilogue<T> epi) {
+__global__ __launch_bounds__(CONV_THREADS, 3) void convMfmaKernel(const half_t* __restrict__ x, int cinStride, int cinPad, int cout,
+                                                               const half_t* __restrict__ w, BoardGeom g, ConvEpilogue<half_t> epi) {
+  using T = half_t;
   using Cfg = MfmaCfg<T>;
   constexpr int BM = CONV_BM;
   constexpr int BK = Cfg::BK;
@@ -1450,14 +1453,14 @@ __global__ void convertToFloatKernel(const T* __restrict__ src, float* __restric
   if(i < n) dst[i] = (float)src[i];
 }
 
-template<typename T, int KS, int BN, int WM>
-void launchMfma(const T* x, int cinStride, int cinPad, int cout, const T* w, BoardGeom g, const ConvEpilogue<T>& epi,
+template<int KS, int BN, int WM>
+void launchMfma(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g, const ConvEpilogue<half_t>& epi,
                 hipStream_t stream) {
-  static const std::string name = kernelLabel("convMfmaKernel<%s, %dx%d, BN=%d, 128-row tiles>", typeLabel<T>(), KS, KS, BN);
+  static const std::string name = kernelLabel("convMfmaKernel<fp16, %dx%d, BN=%d, 128-row tiles>", KS, KS, BN);
   kgh::g_lastConvKernel = name.c_str();
   int M = g.batch * g.H * g.W;
   dim3 grid((M + CONV_BM - 1) / CONV_BM, cout / BN);
-  hipLaunchKernelGGL((convMfmaKernel<T, KS, BN, WM>), grid, dim3(CONV_THREADS), 0, stream, x, cinStride, cinPad, cout, w, g, epi);
+  hipLaunchKernelGGL((convMfmaKernel<KS, BN, WM>), grid, dim3(CONV_THREADS), 0, stream, x, cinStride, cinPad, cout, w, g, epi);
   KGH_CHECK_LAUNCH();
 }
 
@@ -1731,23 +1734,23 @@ bool variantFits(int v, int ky, int cinStride, int cinPad, int cout, BoardGeom g
   return false;
 }
 
-template<typename T, int KS>
-void launchTileVariant(int v, const T* x, int cinStride, int cinPad, int cout, const T* w, BoardGeom g, const ConvEpilogue<T>& epi,
-                       hipStream_t stream) {
+template<int KS>
+void launchTileVariant(int v, const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
+                       const ConvEpilogue<half_t>& epi, hipStream_t stream) {
   switch(v) {
-    case CONV_TILE_192: launchMfma<T, KS, 192, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); break;
-    case CONV_TILE_128: launchMfma<T, KS, 128, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); break;
-    case CONV_TILE_96: launchMfma<T, KS, 96, 4>(x, cinStride, cinPad, cout, w, g, epi, stream); break;
-    case CONV_TILE_64: launchMfma<T, KS, 64, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); break;
-    default: launchMfma<T, KS, 32, 4>(x, cinStride, cinPad, cout, w, g, epi, stream); break;
+    case CONV_TILE_192: launchMfma<KS, 192, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); break;
+    case CONV_TILE_128: launchMfma<KS, 128, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); break;
+    case CONV_TILE_96: launchMfma<KS, 96, 4>(x, cinStride, cinPad, cout, w, g, epi, stream); break;
+    case CONV_TILE_64: launchMfma<KS, 64, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); break;
+    default: launchMfma<KS, 32, 4>(x, cinStride, cinPad, cout, w, g, epi, stream); break;
   }
 }
 
 void launchVariant(int v, int ky, const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g,
                    const ConvEpilogue<half_t>& epi, hipStream_t stream) {
   if(v >= CONV_TILE_192 && v <= CONV_TILE_32) {
-    if(ky == 3) launchTileVariant<half_t, 3>(v, x, cinStride, cinPad, cout, w, g, epi, stream);
-    else launchTileVariant<half_t, 1>(v, x, cinStride, cinPad, cout, w, g, epi, stream);
+    if(ky == 3) launchTileVariant<3>(v, x, cinStride, cinPad, cout, w, g, epi, stream);
+    else launchTileVariant<1>(v, x, cinStride, cinPad, cout, w, g, epi, stream);
     return;
   }
   switch(v) {
@@ -1777,8 +1780,8 @@ void launchVariant(int v, int ky, const half_t* x, int cinStride, int cinPad, in
   throw KghError(5, "conv: variant does not apply");
 }
 
-template<typename T, int KS>
-bool dispatchMfmaTile(const T* x, int cinStride, int cinPad, int cout, const T* w, BoardGeom g, const ConvEpilogue<T>& epi,
+template<int KS>
+bool dispatchMfmaTile(const half_t* x, int cinStride, int cinPad, int cout, const half_t* w, BoardGeom g, const ConvEpilogue<half_t>& epi,
                       hipStream_t stream) {
   // The widest column tile dividing cout that still gives about three
   // workgroups per CU; at small batches the narrowest one (the tuner picks
@@ -1793,11 +1796,11 @@ bool dispatchMfmaTile(const T* x, int cinStride, int cinPad, int cout, const T* 
     if(rowTiles * (cout / cand) >= 3L * 256) break;
   }
   switch(bn) {
-    case 192: launchMfma<T, KS, 192, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); return true;
-    case 128: launchMfma<T, KS, 128, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); return true;
-    case 96: launchMfma<T, KS, 96, 4>(x, cinStride, cinPad, cout, w, g, epi, stream); return true;
-    case 64: launchMfma<T, KS, 64, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); return true;
-    case 32: launchMfma<T, KS, 32, 4>(x, cinStride, cinPad, cout, w, g, epi, stream); return true;
+    case 192: launchMfma<KS, 192, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); return true;
+    case 128: launchMfma<KS, 128, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); return true;
+    case 96: launchMfma<KS, 96, 4>(x, cinStride, cinPad, cout, w, g, epi, stream); return true;
+    case 64: launchMfma<KS, 64, 2>(x, cinStride, cinPad, cout, w, g, epi, stream); return true;
+    case 32: launchMfma<KS, 32, 4>(x, cinStride, cinPad, cout, w, g, epi, stream); return true;
     default: return false;
   }
 }
@@ -1904,11 +1907,11 @@ void launchConv(const T* x, int cinStride, int cin, int cinPad, int cout, int ky
     else if(mfmaPathOk<T>(cinStride, cinPad, cout, ky, kx, wPrepared, epi)) {
       if(ky == 3 && kx == 3) {
         done = dispatch3x3(x, cinStride, cinPad, cout, (const T*)wPrepared, g, epi, stream);
-        if(!done) done = dispatchMfmaTile<T, 3>(x, cinStride, cinPad, cout, (const T*)wPrepared, g, epi, stream);
+        if(!done) done = dispatchMfmaTile<3>(x, cinStride, cinPad, cout, (const T*)wPrepared, g, epi, stream);
       }
       else if(ky == 1 && kx == 1) {
         done = dispatch1x1Dma(x, cinStride, cinPad, cout, (const T*)wPrepared, g, epi, stream);
-        if(!done) done = dispatchMfmaTile<T, 1>(x, cinStride, cinPad, cout, (const T*)wPrepared, g, epi, stream);
+        if(!done) done = dispatchMfmaTile<1>(x, cinStride, cinPad, cout, (const T*)wPrepared, g, epi, stream);
       }
     }
   }

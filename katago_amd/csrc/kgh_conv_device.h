@@ -20,8 +20,6 @@ std::string kernelLabel(const char* fmt, A... a) {
   return buf;
 }
 
-template<typename T> const char* typeLabel() { return std::is_same<T, half_t>::value ? "fp16" : "fp32"; }
-
 }  // namespace
 
 namespace {
@@ -63,9 +61,6 @@ __device__ __forceinline__ void rowColTile(int colTiles, int& rowTile, int& colT
   colTile = id - rowTile * colTiles;
 }
 
-// Epilogue shared by the matrix-core conv kernels; requires
-// convStageBytes(WM) bytes of LDS at smem and must be reached by every
-// thread of the workgroup (it contains barriers).
 // Calls f(std::integral_constant<int, ACT>()) for the epilogue's activation
 // kind, so the per-element activation is selected at compile time instead of
 // branching on every element.
