@@ -1679,19 +1679,27 @@ bool dispatch1x1Dma(const half_t* x, int cinStride, int cinPad, int cout, const 
     kgh::launchStream(tile, x, cinStride, cinPad, cout, w, g, epi, stream);
     return true;
   }
-  // Too few 384-row tiles to fill most CUs: from 24 tiles of 192 rows, the
-  // 192-row kernel with 64-column tiles (two workgroups per CU; b18c384nbt's
-  // 1x1 convs at 16 to 64 boards 12-20 us vs 18-24 us on the 128-row tile
-  // kernel). Below that, where the streamed kernel does not apply, the whole-K
-  // kernel (one memory round trip per tile; b18c384nbt at 1-8 boards: forwards
-  // 0.09-0.12 ms shorter than on the 128-row tile kernel); else the tile
-  // kernel.
-  if((M + TW_BM - 1) / TW_BM * (cout / 64) < 3 * 128) {
-    if(M < 24L * 192) {
-      if(!allK1x1Fits(cinStride, cinPad, cout, 32, g)) return false;
-      launch1x1AllK(x, cinStride, cinPad, cout, w, g, epi, stream);
+  // Below 24 tiles of 192 rows, where the streamed kernel does not apply: the
+  // 192-row kernel with 128-column tiles from 144 of them (768 -> 4096 gated, 8
+  // boards, 512 tiles, four convs per forward: 667 us, 64 columns 708; 4 boards
+  // of 768 -> 2304, 144: 564, 570; 3 boards, 108: 479, 463), else with 64. Other
+  // column counts: the whole-K kernel (one memory round trip per tile;
+  // b18c384nbt at 1-8 boards: forwards 0.09-0.12 ms shorter than on the 128-row
+  // tile kernel), else the tile kernel.
+  if(M < 24L * 192) {
+    if(cout % 64 == 0) {
+      if(cout % 128 == 0 && (M + 191) / 192 * (cout / 128) >= 144) launch1x1Dma<128, 192>(x, cinStride, cinPad, cout, w, g, epi, stream);
+      else launch1x1Dma<64, 192>(x, cinStride, cinPad, cout, w, g, epi, stream);
       return true;
     }
+    if(!allK1x1Fits(cinStride, cinPad, cout, 32, g)) return false;
+    launch1x1AllK(x, cinStride, cinPad, cout, w, g, epi, stream);
+    return true;
+  }
+  // Too few 384-row tiles to fill most CUs: the 192-row kernel with 64-column
+  // tiles (two workgroups per CU; b18c384nbt's 1x1 convs at 16 to 64 boards
+  // 12-20 us vs 18-24 us on the 128-row tile kernel).
+  if((M + TW_BM - 1) / TW_BM * (cout / 64) < 3 * 128) {
     if(cout % 64 != 0) return false;
     launch1x1Dma<64, 192>(x, cinStride, cinPad, cout, w, g, epi, stream);
     return true;

@@ -552,8 +552,13 @@ void launchStreamParts(const half_t* x, int cinStride, int cinPad, int cout, con
     Stream<3, 1, 1, 1, 2, 9>::launchParts(x, cinStride, cinPad, cout, w, g, epi, partChunks, stream);
 }
 
-// 1x1: every shape below 24 row tiles of 192 (a few boards: t12d384h6 at four,
-// forwards 742 -> 652 us). From there on the DMA kernel takes gated outputs and
+// 1x1: below 24 row tiles of 192 while the 32 x 64 tiles times K, what they
+// re-read of rows and weights, stay below a million (t12d384h6 at four
+// boards, forwards 742 -> 652 us; against the 192-row DMA tiles, us of four convs
+// per forward: 1024 -> 1024 at four boards, 0.75 M, -7; 2048 -> 768 at three,
+// 0.84 M, -16; 768 -> 768 at eight, 0.84 M, +8; 768 -> 2304 at four, 1.3 M,
+// +21, at eight, 2.5 M, +58; 768 -> 4096 gated at eight, 4.5 M, +237). From
+// there on the DMA kernel takes gated outputs and
 // K = 1024 (t12d384h6 at 16 boards); else the line follows K. Up to 192 input
 // channels the streamed kernel is faster at every size: a tile holds all of K
 // in little LDS, many workgroups share a CU, and the residual's load hides
@@ -570,7 +575,10 @@ void launchStreamParts(const half_t* x, int cinStride, int cinPad, int cout, con
 int streamTile1x1(int cinStride, int cinPad, int cout, BoardGeom g, const ConvEpilogue<half_t>& epi) {
   const long M = (long)g.batch * g.H * g.W;
   const long tiles = (M + 31) / 32 * (cout / 64);
-  if(M >= 24L * 192) {
+  if(M < 24L * 192) {
+    if(tiles * cinPad > 1000000) return CONV_AUTO;
+  }
+  else {
     if(epi.glu || cinPad > 384 || tiles > (epi.maskResidualAdd ? 2200 : cinPad > 192 ? 4400 : LONG_MAX)) return CONV_AUTO;
   }
   const int v = cinPad <= 192 && tiles > 512 ? CONV_STREAM1_64 : CONV_STREAM1_32;

@@ -121,9 +121,10 @@ T384 = dataclasses.replace(modelgen.transformer_d384(), name="t2d384", blocks=["
     # post convs of 192 input channels always, pre convs of 384 up to 4400
     # tiles, the heads' conv.
     (_nbt(384, 192), [(16, 19, 5, 2), (128, 19, 5, 2), (160, 19, 3, 2)]),
-    # every GEMM; from 24 tiles of 192 rows no gated one nor K = 1024, [Q|K|V] up
+    # every GEMM up to a million of tiles times K, which leaves out the gated one;
+    # from 24 tiles of 192 rows no gated one nor K = 1024, [Q|K|V] up
     # to 4400 tiles, the masked residual up to 2200; the heads' conv.
-    (T384, [(12, 19, 5, 0), (16, 19, 3, 0), (32, 19, 2, 0), (40, 19, 1, 0)]),
+    (T384, [(4, 19, 5, 0), (12, 19, 4, 0), (16, 19, 3, 0), (32, 19, 2, 0), (40, 19, 1, 0)]),
 ], ids=["nbt", "transformer"])
 def test_built_in_choice_for_1x1_convs(model_dir, arch, cases):
     lm = nn.LoadedModel(modelgen.write_model(arch, 57, f"{model_dir}/{arch.name}-1x1.bin"))
