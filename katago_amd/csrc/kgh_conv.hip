@@ -1547,12 +1547,19 @@ bool dispatch3x3(const half_t* x, int cinStride, int cinPad, int cout, const hal
     // boards, 2 against 5, 822 and 750), a round of the tap-window kernel with
     // 128 columns 3.45 times (256 channels, 280 boards 18x18, 2 against 8: 1099
     // and 1201; 200 boards, 2 against 6: 972 and 884).
-    const long streamRounds = tile == CONV_STREAM3_192 ? rounds((M + 191) / 192 * (cout / 64)) : 0;
+    // The tap-window kernel with 192 columns is as fast as streamed 128-row
+    // tiles, two to a CU, where it fills its rounds (192 channels, 240 tiles: 284
+    // boards 18x18 6954 us per forward of b18c384nbt and 7036; 216 tiles, 256
+    // boards: 6456 and 6242).
+    const long streamRounds = tile == CONV_STREAM3_192 && cinPad > 144 ? rounds((M + 191) / 192 * (cout / 64)) : 0;
+    const long tap192 = tapRows * (cout / 192);
     if(board && wide == 64 && 1.9 * rounds(boards) < streamRounds) launchBoardWindow<64>(x, cinStride, cinPad, cout, w, g, epi, stream);
     else if(board && wide == 128 && 2.75 * rounds(boards) < streamRounds)
       launchBoardWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
     else if(!board && tap && wide == 128 && 3.45 * rounds(tapRows * (cout / 128)) < streamRounds)
       launchTapWindow<128>(x, cinStride, cinPad, cout, w, g, epi, stream);
+    else if(!board && tap && wide == 192 && tile == CONV_STREAM3_128 && tap192 >= 235 * rounds(tap192))
+      launchTapWindow<192>(x, cinStride, cinPad, cout, w, g, epi, stream);
     else kgh::launchStream(tile, x, cinStride, cinPad, cout, w, g, epi, stream);
     return true;
   }

@@ -529,15 +529,23 @@ void launchStream(int variant, const half_t* x, int cinStride, int cinPad, int c
 // channels at 19x19: one board 9.0 / 9.5 / 11.5 / 14.5; 8 boards 11.6 / 9.8 /
 // 11.7 / 14.7; 16 boards 13.7 / 13.6 / 12.1 / 14.8; 32 boards 20.6 / 19.3 /
 // 19.5 / 16.5; 96 boards 44.7 / 38.9 / 35.5 / 42.1; 256 -> 256 channels, 160
-// boards: 97.9 / 89.2 / 87.4 / 80.4.
+// boards: 97.9 / 89.2 / 87.4 / 80.4. Where two workgroups of 192 rows fit too
+// (up to 144 channels), they are taken if their rounds of the CUs' 512 places
+// take fewer rows (64 -> 64, sixteen convs per forward: 192 boards, 1 against 2
+// rounds, 394 and 418; 160 boards, 1 and 1, 363 and 329; 128 -> 128, 96 boards,
+// 1 and 2, 442 and 468; 160 boards, 2 and 2, 655 and 626).
 int streamTile3x3(int cinStride, int cinPad, int cout, BoardGeom g, const ConvEpilogue<half_t>& epi) {
   const long M = (long)g.batch * g.H * g.W;
   const std::pair<int, int> tiles[] = {{CONV_STREAM3_32, 32}, {CONV_STREAM3_64, 64}, {CONV_STREAM3_128, 128}, {CONV_STREAM3_192, 192}};
   for(const auto& t : tiles)
     if((M + t.second - 1) / t.second * (cout / 64) <= 256 && streamFits(t.first, cinStride, cinPad, cout, g, epi)) return t.first;
-  if(streamFits(CONV_STREAM3_128, cinStride, cinPad, cout, g, epi) && streamLdsBytes<3, 128, 4>(cinPad, g.W) <= STREAM_MAX_LDS / 2)
-    return CONV_STREAM3_128;
-  if(streamFits(CONV_STREAM3_192, cinStride, cinPad, cout, g, epi)) return CONV_STREAM3_192;
+  const bool fits192 = streamFits(CONV_STREAM3_192, cinStride, cinPad, cout, g, epi);
+  if(streamFits(CONV_STREAM3_128, cinStride, cinPad, cout, g, epi) && streamLdsBytes<3, 128, 4>(cinPad, g.W) <= STREAM_MAX_LDS / 2) {
+    auto roundRows = [&](int rows) { return ((M + rows - 1) / rows * (cout / 64) + 511) / 512 * rows; };
+    const bool two192 = fits192 && streamLdsBytes<3, 192, 4>(cinPad, g.W) <= STREAM_MAX_LDS / 2;
+    return two192 && roundRows(192) < roundRows(128) ? CONV_STREAM3_192 : CONV_STREAM3_128;
+  }
+  if(fits192) return CONV_STREAM3_192;
   return CONV_AUTO;
 }
 

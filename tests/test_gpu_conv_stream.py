@@ -64,8 +64,10 @@ def test_every_tile_gives_the_tile_kernels_bits(model_dir, arch):
 
 
 # Channels, then (boards, side, what the kernel's name holds) on both sides of
-# the lines that the built-in choice draws for 3x3 convs of 224 channels and more.
+# the lines that the built-in choice draws for 3x3 convs.
 CHOICES = [
+    (64, [(160, 19, "128x64 tiles"), (192, 19, "192x64 tiles")]),
+    (192, [(256, 18, "128x64 tiles"), (284, 18, "convTapWindowKernel<3x3 fp16, BN=192")]),
     (256, [(64, 19, "192x64 tiles"), (80, 19, "BN=128, one board"), (200, 13, "192x64 tiles"), (256, 13, "convTapWindowKernel<3x3 fp16, BN=128")]),
     (320, [(80, 19, "192x64 tiles"), (96, 19, "BN=64, one board")]),
     (384, [(14, 19, "128x64 tiles"), (16, 19, "half a board per workgroup, 32-row"), (24, 19, "128x64 tiles"), (32, 19, "BN=64, one board"),
@@ -101,7 +103,7 @@ def _run(model, n, x, kind):
 
 
 @pytest.mark.parametrize("c,choices", CHOICES, ids=lambda v: str(v) if isinstance(v, int) else "")
-def test_built_in_choice_for_wide_convs(model_dir, c, choices):
+def test_built_in_choice_for_3x3_convs(model_dir, c, choices):
     """The kernel that measured fastest runs, and gives the tile kernel's bits."""
     lm = nn.LoadedModel(modelgen.write_model(_block(c), 57, f"{model_dir}/block{c}.bin"))
     model = nn.DeviceModel(lm, use_fp16=True)
