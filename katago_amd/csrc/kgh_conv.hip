@@ -1972,10 +1972,10 @@ void launchConvSplitK(const half_t* x, int cinStride, int cinPad, int cout, cons
   // The streamed kernel adds the splits' sums in registers, the same sums in
   // the same order as split-K workgroups and a second launch, wherever its
   // 64-row tile fits the LDS (up to 704 channels). us per forward of four
-  // blocks, in registers / split-K: 448 channels 158 / 169 at one board, 367 /
-  // 465 at 16; 640: 191 / 197, 624 / 698; 704: 202 / 195, 688 / 819; 768, with
-  // 32-row tiles one to a CU: 214 / 209, 1229 / 959. (b18c384nbt at one board:
-  // 836 / 1055 before the streamed kernels.)
+  // blocks, in registers / split-K: 448 channels 157 / 169 at one board, 358 /
+  // 468 at 16; 640: 190 / 197, 615 / 694; 704: 202 / 195, 203 / 248 at two, 684
+  // / 822 at 16; 768, with 32-row tiles one to a CU: 214 / 210, 1229 / 957.
+  // (b18c384nbt at one board: 812, before the streamed kernels 1054.)
   if(kgh::streamFits(CONV_STREAM3_64, cinStride, cinPad, cout, g, epi)) {
     kgh::launchStreamParts(x, cinStride, cinPad, cout, w, g, epi, splitKChunks(cinPad), stream);
     return;

@@ -47,8 +47,10 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // round trip), split, products, sum, store, of which the products are a third;
 // at 64 boards they are 0.45 of the time. us per launch against 32 x 32 blocks
 // of v_mfma_f32_32x32x2_f32, 192 -> 192 channels at 19x19: 1 board 17.5 ->
-// 15.3, 16 boards 59 -> 29, 64 boards 183 -> 92. Mean error of b18c384nbt's
-// outputs against float64 2.6e-6 -> 7e-7 of their range.
+// 15.3, 16 boards 59 -> 29, 64 boards 183 -> 92. Errors against float64, in the
+// 2-norm: of one conv 0.5e-7 to 1.7e-7 (numpy's fp32 sums 1.2e-7 to 3.6e-7); of
+// b18c384nbt's outputs at 16 boards, the worst one, 4.7e-7 to 6.7e-7 over five
+// seeds, 2.1e-6 to 2.4e-6 on v_mfma_f32_32x32x2_f32.
 constexpr int SPLIT_GROUPS = 4;
 constexpr int SPLIT_STAGE_BYTES = 32 * CONV_STAGE_LD * 4;  // a wave's epilogue stage
 constexpr int SPLIT_PART_BYTES = 16 * 64 * 4;              // a wave's partial sums of one 32 x 32 block

@@ -142,10 +142,10 @@ __device__ __forceinline__ void storeWaveRows(floatx16 (&acc)[RB][CB], float* st
 
 // PARTS (3x3, low-latency mode): every partChunks 32-channel chunks have a sum
 // of their own, started at zero; the sums are added in order, then the bias
-// and the residual. Additions after each part wait for the matrix core, ~1 us
-// of a launch of 7.6 us at 192 channels and one board; a second set of
-// accumulators, added and cleared during the next part's instructions, was
-// slower (the forward 861 us against 836).
+// and the residual. Additions after each part wait for the matrix core: 0.7 us
+// of 7.4 at 192 channels and one board (b18c384nbt's forward 812 us, 762 with
+// one sum); a second set of accumulators, added and cleared during the next
+// part's instructions, was slower (861 us where this form took 836).
 template<int KS, int RB, int CB, int WM, int WN, int DEPTH, bool GLU, bool PARTS>
 __global__ __launch_bounds__(64 * WM * WN, 1) void convStreamKernel(const half_t* __restrict__ x, int cinStride, int cinPad, int cout,
                                                                     const half_t* __restrict__ wf, BoardGeom g, StreamDims sd,
