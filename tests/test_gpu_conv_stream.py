@@ -115,6 +115,8 @@ def test_built_in_choice_for_3x3_convs(model_dir, c, choices):
         h.close()
 
 
+T768 = dataclasses.replace(modelgen.transformer_d384(), name="t2d768", trunk_c=768, mid_c=768, heads=12, kv_heads=12, ffn_c=2048,
+                           blocks=["attention", "ffn"])
 T384 = dataclasses.replace(modelgen.transformer_d384(), name="t2d384", blocks=["attention", "ffn"])
 
 
@@ -127,7 +129,10 @@ T384 = dataclasses.replace(modelgen.transformer_d384(), name="t2d384", blocks=["
     # from 24 tiles of 192 rows no gated one nor K = 1024, [Q|K|V] up
     # to 4400 tiles, the masked residual up to 2200; the heads' conv.
     (T384, [(4, 19, 5, 0), (12, 19, 4, 0), (16, 19, 3, 0), (32, 19, 2, 0), (40, 19, 1, 0)]),
-], ids=["nbt", "transformer"])
+    # wide GEMMs: the gated one from two boards, [Q|K|V] and linear2 from eight
+    # and the output projection from twelve are past a million.
+    (T768, [(2, 19, 4, 0), (8, 19, 2, 0), (12, 19, 1, 0)]),
+], ids=["nbt", "transformer", "wide-transformer"])
 def test_built_in_choice_for_1x1_convs(model_dir, arch, cases):
     lm = nn.LoadedModel(modelgen.write_model(arch, 57, f"{model_dir}/{arch.name}-1x1.bin"))
     model = nn.DeviceModel(lm, use_fp16=True)
